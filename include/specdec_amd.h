@@ -274,10 +274,11 @@ int sd_paged_attention_store(const void* key, int64_t key_stride_tok, int64_t ke
                              size_t workspace_bytes, int32_t num_splits, void* stream);
 
 /*
- * Bytes of workspace that sd_w8a16_linear needs for this shape. Always 0 in
- * this implementation (one launch; K splits are reduced inside a workgroup);
- * the query and the workspace arguments stay in the ABI so callers need not
- * change if a shape ever needs scratch memory.
+ * Bytes of workspace that sd_w8a16_linear uses for this shape on the current
+ * device: the fp32 partial sums of the K slices where more than 16 rows have
+ * too few output tiles to fill the device, 0 for every other shape. The scratch
+ * must be 16-byte aligned. Without it (NULL or too small) the call still runs,
+ * in one slice, and is slower.
  */
 size_t sd_w8a16_workspace_size(int64_t M, int64_t N, int64_t K, int32_t group_size);
 
@@ -296,8 +297,9 @@ size_t sd_w8a16_workspace_size(int64_t M, int64_t N, int64_t K, int32_t group_si
  * per-channel scale on weights up to 32 MiB (M * ceil(K / 1024) <= 4) stream
  * whole weight rows through fp32 FMAs, and so does one row on larger weights
  * (the lm_head), with batches of 4 rows dealt to the waves in turn; other
- * shapes run the MFMA kernel (the SiLU and RMSNorm forms below follow the
- * same rule). Supported: K % 64 == 0,
+ * shapes run the 16-row MFMA kernel (the SiLU and RMSNorm forms below follow the
+ * same rule), and past 16 rows most run a tiled MFMA kernel (small layers at
+ * up to 128 rows stay on the former). Supported: K % 64 == 0,
  * group_size 0 or a multiple of 64 dividing K; N < 2^24 rows, a row stride
  * below 2^24 bytes and N * w_stride_n < 2^32 bytes (the MFMA kernel forms a
  * row's byte offset with one 24 x 24-bit multiply-add; SD_ERR_UNSUPPORTED

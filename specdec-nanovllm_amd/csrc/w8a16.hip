@@ -23,14 +23,10 @@
 // (narrow layers such as N = 1024). One or two activation rows on matrices up
 // to 32 MiB take the row-streaming kernel instead (w8a16_rows_kernel: whole
 // weight rows per load, activations in registers, no MFMA or LDS).
-//
-// int8 -> fp16: (b ^ 0x80) in the low byte under exponent byte 0x64 is the
-// fp16 value 1024 + b + 128, exact; subtracting 1152 (packed fp16) gives b.
-// int8 -> bf16: v_cvt_f32_ubyte of (b ^ 0x80) minus 128 is b as fp32, whose
-// upper half is the exact bf16 (|b| <= 127 needs 7 mantissa bits).
+// Past 16 rows most shapes run the many-row kernel (w8a16_gemm.hip).
 #include <mutex>
 
-#include "sd_common.h"
+#include "w8a16.h"
 
 namespace {
 
@@ -70,46 +66,8 @@ struct W8Params {
   int32_t pair;
 };
 
-__device__ __forceinline__ float load_scale(const void* s, int dtype, int64_t i) {
-  if (dtype == SD_F32) return static_cast<const float*>(s)[i];
-  const uint16_t b = static_cast<const uint16_t*>(s)[i];
-  return dtype == SD_BF16 ? sd::from_bits<__bf16>(b) : sd::from_bits<_Float16>(b);
-}
-
-// 8 int8 (two dwords) -> 8 x 16-bit floats in MFMA operand order.
-template <typename T> __device__ __forceinline__ u32x4 dequant8(uint32_t w0, uint32_t w1);
-
-template <> __device__ __forceinline__ u32x4 dequant8<_Float16>(uint32_t w0, uint32_t w1) {
-  const uint32_t u0 = w0 ^ 0x80808080u, u1 = w1 ^ 0x80808080u;
-  const sd::f16x2 off = {static_cast<_Float16>(1152.f), static_cast<_Float16>(1152.f)};
-  u32x4 r;
-  r.x = __builtin_bit_cast(uint32_t,
-                           __builtin_bit_cast(sd::f16x2, __builtin_amdgcn_perm(0x64646464u, u0, 0x04010400u)) - off);
-  r.y = __builtin_bit_cast(uint32_t,
-                           __builtin_bit_cast(sd::f16x2, __builtin_amdgcn_perm(0x64646464u, u0, 0x04030402u)) - off);
-  r.z = __builtin_bit_cast(uint32_t,
-                           __builtin_bit_cast(sd::f16x2, __builtin_amdgcn_perm(0x64646464u, u1, 0x04010400u)) - off);
-  r.w = __builtin_bit_cast(uint32_t,
-                           __builtin_bit_cast(sd::f16x2, __builtin_amdgcn_perm(0x64646464u, u1, 0x04030402u)) - off);
-  return r;
-}
-
-__device__ __forceinline__ uint32_t bf16_pair(uint32_t u, int lo_byte) {
-  const float a = static_cast<float>((u >> (8 * lo_byte)) & 0xffu) - 128.f;
-  const float b = static_cast<float>((u >> (8 * lo_byte + 8)) & 0xffu) - 128.f;
-  return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, a),
-                               0x07060302u);
-}
-
-template <> __device__ __forceinline__ u32x4 dequant8<__bf16>(uint32_t w0, uint32_t w1) {
-  const uint32_t u0 = w0 ^ 0x80808080u, u1 = w1 ^ 0x80808080u;
-  u32x4 r;
-  r.x = bf16_pair(u0, 0);
-  r.y = bf16_pair(u0, 2);
-  r.z = bf16_pair(u1, 0);
-  r.w = bf16_pair(u1, 2);
-  return r;
-}
+using sd::dequant8;
+using sd::load_scale;
 
 // Row groups of 16 NT rows are spread over the grid (grid-stride). KW waves
 // share one row group and split its K (partials meet in LDS); with KW == 1 the
@@ -1267,10 +1225,12 @@ struct RowsPlan {
 
 struct W8Plan {
   int MT, NT, KW, mblocks, groups, grid;
+  int gemm;  // K slices of the many-row kernel (plain calls run it), 0: it stays out
 };
 
-W8Plan make_plan(int64_t M, int64_t N, int64_t K) {
+W8Plan make_plan(int64_t M, int64_t N, int64_t K, int32_t group) {
   W8Plan pl;
+  pl.gemm = sd::w8a16_gemm_splits(M, N, K, group);
   // Activation rows in blocks of 16 (MT = 1), 32 (MT = 2) or 64 (MT = 4) along
   // grid.y. Every block streams the whole weight matrix, and a second block
   // only hits L2 while it runs in step with the first: with the weight loads
@@ -1288,7 +1248,9 @@ W8Plan make_plan(int64_t M, int64_t N, int64_t K) {
   // 8 when that keeps at most about 16 waves per CU busy with whole 2-step
   // chunks each (a narrow layer has too few tiles to fill the GPU with 4:
   // N = 1024 is 64 workgroups), else 4.
-  if (nr * pl.mblocks >= 8ll * cus || nks < 4) {
+  // Where plain calls run the many-row kernel, the SiLU and RMSNorm forms keep to its
+  // K slices (the same sums).
+  if (pl.gemm == 1 || (pl.gemm == 0 && (nr * pl.mblocks >= 8ll * cus || nks < 4))) {
     pl.KW = 1;
     // 16-row groups balance better over the waves (lm_head M = 1: 29.0 vs
     // 30.0 us); from M = 8 up, 32-row groups reuse each activation read twice
@@ -1299,7 +1261,8 @@ W8Plan make_plan(int64_t M, int64_t N, int64_t K) {
     pl.mblocks = static_cast<int>((M + 15) / 16);
     const int64_t tiles = nr * pl.mblocks;
     // (whole 2-step chunks per wave: a partial chunk loads steps nobody uses)
-    pl.KW = tiles * 16 <= 16ll * cus && nks % 32 == 0 ? 16
+    pl.KW = pl.gemm > 1 ? pl.gemm
+            : tiles * 16 <= 16ll * cus && nks % 32 == 0 ? 16
             : (tiles * 8 <= 16ll * cus && nks % 16 == 0 ? 8 : 4);
   }
   pl.groups = static_cast<int>((nr + pl.NT - 1) / pl.NT);
@@ -1458,6 +1421,7 @@ int launch_all(const W8Params& p, const W8Plan& pl, hipStream_t st) {
   if (p.group == 0) {
     switch (pl.KW) {
       case 1: rc = launch_kw<T, false, 1, MODE, FLOOR>(p, pl, grid, st); break;
+      case 2: rc = launch_kw<T, false, 2, MODE, FLOOR>(p, pl, grid, st); break;
       case 16: rc = launch_kw<T, false, 16, MODE, FLOOR>(p, pl, grid, st); break;
       case 8: rc = launch_kw<T, false, 8, MODE, FLOOR>(p, pl, grid, st); break;
       default: rc = launch_kw<T, false, 4, MODE, FLOOR>(p, pl, grid, st); break;
@@ -1469,6 +1433,7 @@ int launch_all(const W8Params& p, const W8Plan& pl, hipStream_t st) {
     } else {
       switch (pl.KW) {
         case 1: rc = launch_kw<T, true, 1, MODE>(p, pl, grid, st); break;
+        case 2: rc = launch_kw<T, true, 2, MODE>(p, pl, grid, st); break;
         case 16: rc = launch_kw<T, true, 16, MODE>(p, pl, grid, st); break;
         case 8: rc = launch_kw<T, true, 8, MODE>(p, pl, grid, st); break;
         default: rc = launch_kw<T, true, 4, MODE>(p, pl, grid, st); break;
@@ -1592,11 +1557,10 @@ int launch_rows_any(const W8Params& p, int mode, hipStream_t st) {
 }  // namespace
 
 extern "C" size_t sd_w8a16_workspace_size(int64_t M, int64_t N, int64_t K, int32_t group_size) {
-  (void)M;
-  (void)N;
-  (void)K;
-  (void)group_size;
-  return 0;  // one launch; K splits are reduced inside the workgroup
+  if (M <= 0 || N <= 0 || K <= 0 || K % 64 || group_size < 0 || group_size % 64 || M > (1ll << 30) ||
+      N > (1ll << 30) || K > (1ll << 30) || (group_size && K % group_size))
+    return 0;  // nothing to run, or refused by sd_w8a16_linear
+  return sd::w8a16_gemm_workspace(M, N, K, group_size);
 }
 
 namespace {
@@ -1619,7 +1583,7 @@ int run_w8a16(const void* x, int64_t x_stride_m, int64_t up, const NormArgs& nor
               const int8_t* w, int64_t w_stride_n, const void* scale, int32_t scale_dtype,
               int32_t group_size, const void* bias, void* y, int64_t y_stride_m, int64_t M,
               int64_t N, int64_t K, int32_t dtype, void* stream, bool pair = false,
-              bool floor = false) {
+              bool floor = false, void* workspace = nullptr, size_t workspace_bytes = 0) {
   if (M < 0 || N <= 0 || K <= 0 || group_size < 0) {
     sd::set_error("w8a16: invalid sizes M=%lld N=%lld K=%lld group=%d", (long long)M,
                   (long long)N, (long long)K, group_size);
@@ -1686,7 +1650,7 @@ int run_w8a16(const void* x, int64_t x_stride_m, int64_t up, const NormArgs& nor
                   "still read the inputs)");
     return SD_ERR_VALUE;
   }
-  const W8Plan pl = make_plan(M, N, K);
+  const W8Plan pl = make_plan(M, N, K, group_size);
   W8Params p;
   p.x = static_cast<const uint16_t*>(x);
   p.xs = x_stride_m;
@@ -1723,7 +1687,7 @@ int run_w8a16(const void* x, int64_t x_stride_m, int64_t up, const NormArgs& nor
     // the plain projection's plan (same K split, so the same sums), per-channel
     // scales and whole 16-row tiles of pairs
     const bool rows = N % 2 == 0 && rows_eligible(p, true);
-    const bool tiled = N % 32 == 0 && pl.KW > 1 && group_size == 0 && mode != 1;
+    const bool tiled = N % 32 == 0 && pl.KW > 1 && pl.gemm == 0 && group_size == 0 && mode != 1;
     if (!rows && !tiled) {
       sd::set_error("w8a16_gate_up_silu: the SiLU epilogue runs on the row-streaming path "
                     "(one or two rows, M * ceil(K / 1024) <= 4, per-channel scales, at most "
@@ -1749,6 +1713,13 @@ int run_w8a16(const void* x, int64_t x_stride_m, int64_t up, const NormArgs& nor
     }
     if (dtype == SD_BF16) return launch_all<__bf16, 0>(p, pp, st);
     return launch_all<_Float16, 0>(p, pp, st);
+  }
+  if (pl.gemm > 0 && mode == 0) {
+    const sd::W8GemmArgs ga{p.x, p.xs, p.w, p.ws, p.scale, p.scale_dtype, p.group, p.bias,
+                            p.y, p.ys, p.M, p.N,  p.K,     dtype};
+    int splits = 0;
+    if (sd::w8a16_gemm_fits(ga, workspace, workspace_bytes, &splits))
+      return sd::w8a16_gemm(ga, splits, workspace, st, floor);
   }
   if (floor) {  // the plain form's plan with the load-only kernels
     if (rows_eligible(p, false)) {
@@ -1782,10 +1753,9 @@ extern "C" int sd_w8a16_linear(const void* x, int64_t x_stride_m, const int8_t* 
                                int64_t M, int64_t N, int64_t K, int32_t dtype, void* workspace,
                                size_t workspace_bytes, void* stream) {
   sd::clear_error();
-  (void)workspace;
-  (void)workspace_bytes;
   return run_w8a16(x, x_stride_m, -1, NormArgs{}, w, w_stride_n, scale, scale_dtype, group_size,
-                   bias, y, y_stride_m, M, N, K, dtype, stream);
+                   bias, y, y_stride_m, M, N, K, dtype, stream, false, false, workspace,
+                   workspace_bytes);
 }
 
 extern "C" int sd_w8a16_floor(const void* x, int64_t x_stride_m, const int8_t* w,

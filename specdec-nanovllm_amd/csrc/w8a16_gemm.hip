@@ -1,0 +1,495 @@
+// w8a16_gemm.hip — the W8A16 linear over many activation rows (prefill, verify
+// and decode batches past 16 rows) for gfx950: an MFMA GEMM that dequantizes the
+// int8 weights between LDS and the matrix cores.
+//
+//   y[m, n] = scale[n] * sum_k x[m, k] * w[n, k] (+ bias[n])           per channel
+//   y[m, n] = sum_g scale[n, g] * sum_{k in g} x[m, k] * w[n, k] (+ bias)  per group
+//
+// Bound: the matrix cores (2 M N K operations against N K + 2 M (N + K) bytes) from
+// about 200 rows up, HBM below. Layout of one step (64 columns of K):
+//  * x rows (128 B) and weight rows (64 B) go from HBM / L2 straight into LDS
+//    (global_load_lds, 16 B per lane, no registers); the 16-byte units of a row are
+//    permuted by the global address of each lane (unit u of x row r lies at position
+//    u ^ (r / 2 & 7), of weight row r at u ^ (r / 4 NT & 3)), so that the 16 lanes of
+//    an operand read hit 16 different 16-byte slots of the 256-byte bank row;
+//  * the weights stay int8 in LDS (half the LDS traffic of a 16-bit tile) and each
+//    wave dequantizes the operands it reads (sd::dequant8): 96 VALU instructions beside
+//    64 MFMAs per wave and step at 128 x 64 outputs per wave;
+//  * the weights are the MFMA A operand. Tile row 4 g + i of tile t is weight row
+//    4 NT g + 4 t + i of the wave, so a lane's sums are 4 NT consecutive outputs of one
+//    row and leave in 16-byte stores.
+// The loop runs half a step ahead: the second half's x operands load under the first
+// half's MFMAs; then one barrier (the next step has landed in every wave's view, this
+// step's LDS is read), the load of step + S into the freed stage, and the next step's
+// first operands under the second half's MFMAs.
+//
+// Sums: one fp32 accumulator per output over the K slice, in ascending k and with the
+// operand order of w8a16_kernel (lane group g holds k = 16 g .. 16 g + 15 of a step, two
+// MFMAs), so a shape gives the same bits on either kernel with the same K slices. With
+// several slices each writes its fp32 partials and w8a16_gemm_reduce adds them in slice
+// order, then scales and rounds (partial sums stay 32-bit).
+#include "w8a16.h"
+
+namespace {
+
+using sd::f32x4;
+using sd::u32x4;
+
+struct GemmParams {
+  sd::W8GemmArgs a;
+  float* part;      // splits > 1: [splits][M][pitch] partial sums
+  int64_t pitch;
+  int32_t nks;      // 64-column steps of the whole K
+  int32_t tiles_m, tiles_n, splits;
+  int32_t vec_out;  // y rows allow 16-byte stores
+};
+
+__device__ __forceinline__ void load_lds16(const void* g, void* l) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)g,
+                                   (__attribute__((address_space(3))) void*)l, 16, 0, 0);
+}
+
+// Wait for all but the newest N vector-memory loads of this wave and for its LDS
+// reads, then for the workgroup.
+template <int N> __device__ __forceinline__ void wait_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// WM x WN waves, each MT x NT tiles of 16 x 16 outputs; S stages of 64 columns.
+template <typename T, int WM, int WN, int MT, int NT, int S, int WPE, bool PG, bool FLOOR>
+__global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
+void w8a16_gemm_kernel(GemmParams p) {
+  constexpr int NW = WM * WN, BM = WM * MT * 16, BN = WN * NT * 16;
+  constexpr int XB = BM * 128, SB = XB + BN * 64;  // bytes of a stage: x rows, weight rows
+  constexpr int CX = BM / 8 / NW, CW = BN / 16 / NW;  // 1 KB loads per wave and stage
+  constexpr int LPW = CX + CW;
+  static_assert(CX * NW * 8 == BM && CW * NW * 16 == BN && NT % 2 == 0, "whole 1 KB loads per wave");
+  extern __shared__ __attribute__((aligned(1024))) char sm[];
+  const sd::W8GemmArgs& a = p.a;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  const int wm = wave / WN, wn = wave % WN;
+
+  // Workgroup -> (slice, tile): every eighth workgroup shares an XCD (one L2), so each
+  // XCD takes a contiguous run of tiles, 8 M tiles deep before the next N tile.
+  const int items = p.tiles_m * p.tiles_n * p.splits;
+  int id = blockIdx.x;
+  {
+    const int per = items / 8, rem = items % 8, xcd = id % 8;
+    id = xcd * per + min(xcd, rem) + id / 8;
+  }
+  const int tiles = p.tiles_m * p.tiles_n;
+  const int slice = id / tiles;
+  id -= slice * tiles;
+  constexpr int kGroupM = 8;
+  const int gi = id / (kGroupM * p.tiles_n), gr = id - gi * kGroupM * p.tiles_n;
+  const int gm = min(kGroupM, p.tiles_m - gi * kGroupM);
+  const int m0 = (gi * kGroupM + gr % gm) * BM, n0 = gr / gm * BN;
+  const int ks = static_cast<int>(static_cast<int64_t>(slice) * p.nks / p.splits);
+  const int ke = static_cast<int>(static_cast<int64_t>(slice + 1) * p.nks / p.splits);
+
+  // ---- loads: this lane's 16-byte unit of each 1 KB (8 x rows, 16 weight rows); rows
+  //      past M / N read the last row (their outputs are not written), steps past the
+  //      slice read its last step (into a stage nobody reads)
+  const char* xbase = reinterpret_cast<const char*>(a.x + static_cast<int64_t>(m0) * a.xs);
+  const char* wbase = reinterpret_cast<const char*>(a.w + static_cast<int64_t>(n0) * a.ws);
+  uint32_t xoff[CX], woff[CW];
+#pragma unroll
+  for (int i = 0; i < CX; ++i) {
+    const int r = (wave * CX + i) * 8 + (lane >> 3), unit = (lane & 7) ^ ((r >> 1) & 7);
+    xoff[i] = static_cast<uint32_t>(min(r, a.M - 1 - m0)) * static_cast<uint32_t>(a.xs * 2) + unit * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < CW; ++i) {
+    const int r = (wave * CW + i) * 16 + (lane >> 2), unit = (lane & 3) ^ ((r / (4 * NT)) & 3);
+    woff[i] = static_cast<uint32_t>(min(r, a.N - 1 - n0)) * static_cast<uint32_t>(a.ws) + unit * 16;
+  }
+  auto issue = [&](int step, int st) {
+    const int s = min(step, ke - 1);
+    const char* xb = xbase + static_cast<int64_t>(s) * 128;
+    const char* wb = wbase + static_cast<int64_t>(s) * 64;
+    char* stage = sm + st * SB;
+#pragma unroll
+    for (int i = 0; i < CX; ++i) load_lds16(xb + xoff[i], stage + (wave * CX + i) * 1024);
+#pragma unroll
+    for (int i = 0; i < CW; ++i) load_lds16(wb + woff[i], stage + XB + (wave * CW + i) * 1024);
+  };
+
+  if constexpr (FLOOR) {  // the loads and barriers alone
+#pragma unroll
+    for (int s = 0; s < S; ++s) issue(ks + s, s);
+    wait_barrier<(S - 1) * LPW>();
+    int st = 0;
+    for (int step = ks; step < ke; ++step) {
+      wait_barrier<(S - 2) * LPW>();
+      issue(step + S, st);
+      st = st + 1 == S ? 0 : st + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    return;
+  }
+
+  const int nb = n0 + wn * NT * 16 + lg * 4 * NT;  // first of this lane's 4 NT outputs per row
+
+  // ---- per-channel scales (and bias) of this lane's outputs, ahead of the loop; per
+  //      group: the slice's table in LDS after the stages, [group][BN] in fp32
+  float sc[PG ? 1 : NT][4];
+  float* tab = reinterpret_cast<float*>(sm + S * SB);
+  const int spg = PG ? a.group / 64 : 1;           // steps per group
+  const int ng = PG ? a.K / a.group : 1, g0 = ks / spg;
+  if constexpr (PG) {
+    const int groups = (ke - 1) / spg - g0 + 1;
+    for (int i = tid; i < BN * groups; i += NW * 64) {
+      const int n = i / groups, g = i - n * groups;
+      tab[g * BN + n] = sd::load_scale(a.scale, a.scale_dtype,
+                                       static_cast<int64_t>(min(n0 + n, a.N - 1)) * ng + g0 + g);
+    }
+  } else if (p.splits == 1) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sc[t][i] = sd::load_scale(a.scale, a.scale_dtype, min(nb + 4 * t + i, a.N - 1));
+  }
+
+  f32x4 acc[NT][MT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  // ---- LDS operand addresses: x row lr of tile m, 16-byte unit 2 lg + half; weight
+  //      row of tile t, unit lg (16 int8: both halves)
+  const int xa = (wm * MT * 16 + lr) * 128 + (((lg * 2) ^ ((lr >> 1) & 7)) * 16);
+  const int wa = XB + (wn * NT * 16 + (lr >> 2) * 4 * NT + (lr & 3)) * 64 + ((lg ^ (lr >> 2)) * 16);
+  u32x4 xf[2][MT], wr[NT];
+  auto read_x = [&](int st, int half) {
+    const char* b = sm + st * SB + (xa ^ (half * 16));
+#pragma unroll
+    for (int m = 0; m < MT; ++m) xf[half][m] = sd::load16(b + m * 2048);
+  };
+  auto read_w = [&](int st) {
+    const char* b = sm + st * SB + wa;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) wr[t] = sd::load16(b + t * 256);
+  };
+
+  int st = 0;
+  if constexpr (PG) {
+    // one partial sum per step, scaled into the accumulators; the loads run S - 1 steps ahead
+#pragma unroll
+    for (int s = 0; s < S - 1; ++s) issue(ks + s, s);
+    for (int step = ks; step < ke; ++step) {
+      wait_barrier<(S - 2) * LPW>();
+      issue(step + S - 1, st == 0 ? S - 1 : st - 1);
+      read_w(st);
+      read_x(st, 0);
+      read_x(st, 1);
+      const float* tg = tab + (step / spg - g0) * BN + (nb - n0);
+      f32x4 gs[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) gs[t] = *reinterpret_cast<const f32x4*>(tg + 4 * t);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        const u32x4 w0 = sd::dequant8<T>(wr[t].x, wr[t].y), w1 = sd::dequant8<T>(wr[t].z, wr[t].w);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+          f32x4 z = {0.f, 0.f, 0.f, 0.f};
+          z = sd::Elem<T>::mfma(w0, xf[0][m], z);
+          z = sd::Elem<T>::mfma(w1, xf[1][m], z);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) acc[t][m][i] += z[i] * gs[t][i];
+        }
+      }
+      st = st + 1 == S ? 0 : st + 1;
+    }
+  } else {
+#pragma unroll
+    for (int s = 0; s < S; ++s) issue(ks + s, s);
+    wait_barrier<(S - 1) * LPW>();
+    read_w(0);
+    read_x(0, 0);
+    for (int step = ks; step < ke; ++step) {
+      u32x4 wd[NT];
+      read_x(st, 1);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) wd[t] = sd::dequant8<T>(wr[t].x, wr[t].y);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[t][m] = sd::Elem<T>::mfma(wd[t], xf[0][m], acc[t][m]);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) wd[t] = sd::dequant8<T>(wr[t].z, wr[t].w);
+      wait_barrier<(S - 2) * LPW>();
+      issue(step + S, st);
+      st = st + 1 == S ? 0 : st + 1;
+      read_w(st);
+      read_x(st, 0);
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[t][m] = sd::Elem<T>::mfma(wd[t], xf[1][m], acc[t][m]);
+    }
+  }
+  // no load of this workgroup may reach LDS after it has ended
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+  // ---- outputs: lane holds y[m0 + 16 (wm MT + m) + lr][nb + 4 t + i]
+  if (p.splits > 1) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const int r = m0 + (wm * MT + m) * 16 + lr;
+      if (r >= a.M) continue;
+      float* dst = p.part + (static_cast<int64_t>(slice) * a.M + r) * p.pitch + nb;
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        if (nb + 4 * t < a.N) *reinterpret_cast<f32x4*>(dst + 4 * t) = acc[t][m];
+    }
+    return;
+  }
+  float bi[NT][4];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bi[t][i] = a.bias ? sd::from_bits<T>(a.bias[min(nb + 4 * t + i, a.N - 1)]) : 0.f;
+  const bool whole = p.vec_out && nb + 4 * NT <= a.N;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int r = m0 + (wm * MT + m) * 16 + lr;
+    if (r >= a.M) continue;
+    uint16_t* dst = a.y + static_cast<int64_t>(r) * a.ys + nb;
+    float v[NT][4];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[t][i] = acc[t][m][i] * (PG ? 1.f : sc[PG ? 0 : t][i]) + bi[t][i];
+    if (whole) {
+#pragma unroll
+      for (int t = 0; t < NT; t += 2)
+        sd::store16(dst + 4 * t, u32x4{sd::pack2<T>(v[t][0], v[t][1]), sd::pack2<T>(v[t][2], v[t][3]),
+                                       sd::pack2<T>(v[t + 1][0], v[t + 1][1]),
+                                       sd::pack2<T>(v[t + 1][2], v[t + 1][3])});
+    } else {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (nb + 4 * t + i < a.N) dst[4 * t + i] = sd::to_bits<T>(v[t][i]);
+    }
+  }
+}
+
+// Partial sums of the K slices, added in slice order, scaled, rounded: one thread per
+// four outputs of a row, every slice's load in flight at once.
+template <typename T, int SPLITS>
+__global__ __launch_bounds__(256) void w8a16_gemm_reduce(GemmParams p) {
+  const sd::W8GemmArgs& a = p.a;
+  const int nq = (a.N + 3) / 4;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= static_cast<int64_t>(a.M) * nq) return;
+  const int m = static_cast<int>(i / nq), n = static_cast<int>(i - static_cast<int64_t>(m) * nq) * 4;
+  const float* src = p.part + static_cast<int64_t>(m) * p.pitch + n;
+  const int64_t slice = static_cast<int64_t>(a.M) * p.pitch;
+  f32x4 v[SPLITS];
+#pragma unroll
+  for (int s = 0; s < SPLITS; ++s) v[s] = *reinterpret_cast<const f32x4*>(src + s * slice);
+  float sc[4], bi[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int c = min(n + e, a.N - 1);
+    sc[e] = a.group ? 1.f : sd::load_scale(a.scale, a.scale_dtype, c);
+    bi[e] = a.bias ? sd::from_bits<T>(a.bias[c]) : 0.f;
+  }
+  f32x4 acc = v[0];
+#pragma unroll
+  for (int s = 1; s < SPLITS; ++s) acc += v[s];
+  float o[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) o[e] = acc[e] * sc[e] + bi[e];
+  uint16_t* dst = a.y + static_cast<int64_t>(m) * a.ys + n;
+  if (p.vec_out && n + 4 <= a.N) {
+    *reinterpret_cast<uint2*>(dst) = make_uint2(sd::pack2<T>(o[0], o[1]), sd::pack2<T>(o[2], o[3]));
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < a.N) dst[e] = sd::to_bits<T>(o[e]);
+  }
+}
+
+// ------------------------------------------------------------------- launches
+enum Tile { kT64x128, kT128x128, kT128x256, kT256x256 };
+
+struct Shape {
+  int bm, bn;
+};
+constexpr Shape kShapes[] = {{64, 128}, {128, 128}, {128, 256}, {256, 256}};
+
+int64_t tiles_of(Tile t, int64_t M, int64_t N) {
+  return ((M + kShapes[t].bm - 1) / kShapes[t].bm) * ((N + kShapes[t].bn - 1) / kShapes[t].bn);
+}
+
+int64_t pitch_of(int64_t N) { return (N + 3) / 4 * 4; }
+
+// What a tile costs, in microseconds per 64-column step, measured at 256 CUs (M 17 - 4096;
+// N x K 1024 x 2048 to 19456 x 2560 and 151936 x 1024): `alone` with at most one workgroup
+// per CU, `full` per workgroup of a CU that always has more (4096 x 19456 x 2560: 520, 409,
+// 388, 361 us with the four tiles). Per group the step sums and scales come on top, and the
+// tiles stop at 64 x 64 outputs per wave.
+struct Cost {
+  Tile tile;
+  double alone, full;
+};
+constexpr Cost kCosts[] = {{kT64x128, 0.44, 0.341}, {kT128x128, 0.63, 0.535},
+                           {kT128x256, 0.95, 1.01}, {kT256x256, 1.38, 1.78}};
+constexpr Cost kCostsGroup[] = {{kT64x128, 0.55, 0.425}, {kT128x128, 1.2, 0.72}};
+
+struct Plan {
+  Tile tile;
+  int splits;
+};
+
+// The tile and the K slices of least estimated time: rounds of workgroups per CU (between
+// the mean and the largest share: workgroups of a CU run together), about three steps to
+// fill and drain a tile, and for several slices the second launch and the partial sums
+// through memory (4.3 TB/s). Checked against the measured best of all tiles and slices at
+// the sizes above: within 10% of it.
+Plan plan_for(int64_t M, int64_t N, int64_t K, int32_t group) {
+  const int64_t nks = K / 64;
+  const double cus = sd::device_cus();
+  Plan best{kT64x128, 1};
+  double best_us = 1e30;
+  const Cost* costs = group ? kCostsGroup : kCosts;
+  const int ncosts = group ? 2 : 4;
+  for (int c = 0; c < ncosts; ++c)
+    for (int splits = 1; splits <= 16; splits *= 2) {
+      if (splits > 1 && nks < 4 * splits) break;
+      const double n = static_cast<double>(tiles_of(costs[c].tile, M, N)) * splits / cus;
+      const double whole = static_cast<double>(static_cast<int64_t>(n)) + (n > static_cast<int64_t>(n) ? 1 : 0);
+      const double shared = n > 1 ? 0.5 * (n + whole) * costs[c].full : n * costs[c].full;
+      const double step = shared > costs[c].alone ? shared : costs[c].alone;
+      double us = (static_cast<double>((nks + splits - 1) / splits) + 3) * step;
+      if (splits > 1) us += 3.5 + 8.0 * splits * static_cast<double>(M) * static_cast<double>(N) / 4.3e6;
+      if (us < best_us) {
+        best_us = us;
+        best = Plan{costs[c].tile, splits};
+      }
+    }
+  return best;
+}
+
+// LDS of the per-group scale table of a K slice.
+size_t table_bytes(Tile t, int64_t K, int32_t group, int splits) {
+  if (!group) return 0;
+  const int64_t nks = K / 64, spg = group / 64, per = (nks + splits - 1) / splits;
+  return static_cast<size_t>(kShapes[t].bn) * static_cast<size_t>((per + spg - 2) / spg + 1) * sizeof(float);
+}
+
+template <typename T, int WM, int WN, int MT, int NT, int S, int WPE, bool PG, bool FLOOR>
+int launch(GemmParams p, Tile t, hipStream_t st) {
+  constexpr int BM = WM * MT * 16, BN = WN * NT * 16;
+  p.tiles_m = (p.a.M + BM - 1) / BM;
+  p.tiles_n = (p.a.N + BN - 1) / BN;
+  const size_t lds = static_cast<size_t>(S) * (BM * 128 + BN * 64) +
+                     table_bytes(t, p.a.K, FLOOR ? 0 : p.a.group, p.splits);
+  hipLaunchKernelGGL((w8a16_gemm_kernel<T, WM, WN, MT, NT, S, WPE, PG, FLOOR>),
+                     dim3(static_cast<unsigned>(p.tiles_m * p.tiles_n * p.splits)),
+                     dim3(WM * WN * 64), lds, st, p);
+  return SD_OK;
+}
+
+// Stages: four for the small tile (its loads cover HBM latency with one workgroup per CU:
+// M = 56 of 19456 x 2560 took 23 us with two, 20 with four), two elsewhere (more workgroups
+// per CU measured better than more stages: 128 x 128 at 4096 x 19456 x 2560 398 against 424).
+template <typename T, bool PG, bool FLOOR>
+int launch_tile(Tile t, const GemmParams& p, hipStream_t st) {
+  if constexpr (PG) {
+    if (t == kT64x128) return launch<T, 1, 4, 4, 2, 3, 2, true, FLOOR>(p, t, st);
+    return launch<T, 2, 2, 4, 4, 2, 2, true, FLOOR>(p, t, st);
+  } else {
+    switch (t) {
+      case kT64x128: return launch<T, 1, 4, 4, 2, 4, 2, false, FLOOR>(p, t, st);
+      case kT128x128: return launch<T, 2, 2, 4, 4, 2, 3, false, FLOOR>(p, t, st);
+      case kT128x256: return launch<T, 2, 4, 4, 4, 2, 4, false, FLOOR>(p, t, st);
+      default: return launch<T, 2, 4, 8, 4, 2, 2, false, FLOOR>(p, t, st);
+    }
+  }
+}
+
+template <typename T>
+void launch_reduce(const GemmParams& p, hipStream_t st) {
+  const int64_t n = static_cast<int64_t>(p.a.M) * ((p.a.N + 3) / 4);
+  const dim3 grid(static_cast<unsigned>((n + 255) / 256)), block(256);
+  switch (p.splits) {
+    case 2: hipLaunchKernelGGL((w8a16_gemm_reduce<T, 2>), grid, block, 0, st, p); break;
+    case 4: hipLaunchKernelGGL((w8a16_gemm_reduce<T, 4>), grid, block, 0, st, p); break;
+    case 8: hipLaunchKernelGGL((w8a16_gemm_reduce<T, 8>), grid, block, 0, st, p); break;
+    default: hipLaunchKernelGGL((w8a16_gemm_reduce<T, 16>), grid, block, 0, st, p); break;
+  }
+}
+
+template <typename T>
+int run(Tile t, const GemmParams& p, hipStream_t st, bool floor) {
+  if (floor) return launch_tile<T, false, true>(t, p, st);
+  const int rc = p.a.group ? launch_tile<T, true, false>(t, p, st) : launch_tile<T, false, false>(t, p, st);
+  if (rc != SD_OK || p.splits == 1) return rc;
+  launch_reduce<T>(p, st);
+  return SD_OK;
+}
+
+GemmParams params(const sd::W8GemmArgs& a, int splits, void* workspace) {
+  GemmParams p{};
+  p.a = a;
+  p.part = static_cast<float*>(workspace);
+  p.pitch = pitch_of(a.N);
+  p.nks = a.K / 64;
+  p.splits = splits;
+  p.vec_out = sd::aligned16(a.y) && a.ys % 8 == 0;
+  return p;
+}
+
+}  // namespace
+
+namespace sd {
+
+// From 17 rows up, except where the 16-row kernels measured faster: layers of at most
+// 8 Mi weights while M N K <= 5.4e8 and M <= 128 (one launch, K split inside a workgroup:
+// 1024 x 2048 at M = 56 6.1 us there against 9.2 here, at M = 128 10.0 against 10.5, at
+// M = 256 16.8 against 12.3; 6144 x 1024 at M = 56 9.2 against 11.0, at M = 128 13.6
+// against 12.0). Per group the same line; 2560 x 9728 at M = 17 is 20 us there, 14 here.
+int w8a16_gemm_splits(int64_t M, int64_t N, int64_t K, int32_t group) {
+  if (M <= 16) return 0;
+  if (M <= 128 && N * K <= (int64_t{8} << 20) && static_cast<double>(M) * N * K <= 5.4e8) return 0;
+  return plan_for(M, N, K, group).splits;
+}
+
+size_t w8a16_gemm_workspace(int64_t M, int64_t N, int64_t K, int32_t group) {
+  const int splits = w8a16_gemm_splits(M, N, K, group);
+  if (splits <= 1) return 0;
+  return static_cast<size_t>(splits) * static_cast<size_t>(M) * static_cast<size_t>(pitch_of(N)) * sizeof(float);
+}
+
+bool w8a16_gemm_fits(const W8GemmArgs& a, const void* workspace, size_t workspace_bytes, int* splits) {
+  *splits = w8a16_gemm_splits(a.M, a.N, a.K, a.group);
+  if (*splits == 0) return false;
+  // without the partial sums' workspace: one slice
+  if (*splits > 1 && (!workspace || !aligned16(workspace) ||
+                      workspace_bytes < w8a16_gemm_workspace(a.M, a.N, a.K, a.group)))
+    *splits = 1;
+  // a tile's x rows within 32-bit byte offsets; its LDS; the grid
+  const Tile t = plan_for(a.M, a.N, a.K, a.group).tile;
+  if (a.xs >= (int64_t{1} << 23)) return false;
+  if (tiles_of(t, a.M, a.N) * *splits > 0x7fffffff) return false;
+  const size_t stages = t == kT64x128 ? 3 : 2;  // (per group; the others have no table)
+  return !a.group || stages * (kShapes[t].bm * 128 + kShapes[t].bn * 64) +
+                             table_bytes(t, a.K, a.group, *splits) <=
+                         static_cast<size_t>(device_lds_per_block());
+}
+
+int w8a16_gemm(const W8GemmArgs& a, int splits, void* workspace, hipStream_t st, bool floor) {
+  const Tile t = plan_for(a.M, a.N, a.K, a.group).tile;
+  const GemmParams p = params(a, splits, workspace);
+  const int rc = a.dtype == SD_BF16 ? run<__bf16>(t, p, st, floor) : run<_Float16>(t, p, st, floor);
+  return rc != SD_OK ? rc : check_launch(floor ? "w8a16 floor" : "w8a16");
+}
+
+}  // namespace sd

@@ -338,8 +338,10 @@ def w8a16_silu_linear(gate_up: torch.Tensor, qweight: torch.Tensor, scale: torch
     """w8a16_linear(silu_mul(gate_up), ...): the MLP's act_fn and down_proj
     (layers/activation.py:6-11 then the W8A16 linear). gate_up: (..., 2K); the
     activation is SiluAndMul's, bit for bit. One launch while the fused form
-    stages its activation rows in LDS (min(M, 16) (2K + 16) <= 33,024 bytes),
-    the two separate launches otherwise (the faster of the two there)."""
+    stages its activation rows in LDS (min(M, 16) (2K + 16) <= 33,024 bytes)
+    and the plain linear stays on the 16-row kernels it shares (up to 16 rows,
+    or 128 on at most 8 Mi weights), the two separate launches otherwise (the
+    faster of the two there)."""
     assert qweight.dtype == torch.int8 and qweight.dim() == 2
     N, K = qweight.shape
     g2 = gate_up.reshape(-1, gate_up.shape[-1])
@@ -353,7 +355,7 @@ def w8a16_silu_linear(gate_up: torch.Tensor, qweight: torch.Tensor, scale: torch
         assert sc.numel() == N * (K // group_size), "per-group scale must be (N, K // group_size)"
     else:
         assert sc.numel() == N, "per-channel scale must have N entries"
-    if min(M, 16) * (2 * K + 16) > 33024:
+    if min(M, 16) * (2 * K + 16) > 33024 or M > (16 if N * K > 8 << 20 else 128):
         y = w8a16_linear(silu_mul(g2), qw, sc, bias, group_size, out)
         return y.view(*gate_up.shape[:-1], N)
     b = None if bias is None else bias.to(gate_up.dtype).contiguous()

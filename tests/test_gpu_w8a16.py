@@ -358,6 +358,61 @@ def test_gate_up_silu_entry_refuses_shapes_off_its_paths():
     assert rc == _lib.SD_ERR_UNSUPPORTED and b"row-streaming" in lib.sd_last_error()
 
 
+# ------------------------------------------------------------- many rows
+@pytest.mark.parametrize("M,N,K,gs", [(17, 9000, 1024, 0),      # 64 x 128 tiles, a ragged last one
+                                      (65, 16400, 640, 0),      # one row into the second tile
+                                      (129, 2560, 4096, 0),     # K slices, added by the second launch
+                                      (200, 1030, 2048, 128),   # the same per group, N % 4 != 0
+                                      (300, 6144, 1024, 64),    # one scale per step
+                                      (257, 24200, 192, 0),     # three steps
+                                      (1025, 12290, 64, 0),     # a single step, odd outputs
+                                      (2049, 8200, 256, 0),     # 128 x 256 and 256 x 256 tiles
+                                      (4097, 9728, 128, 256)])
+@pytest.mark.parametrize("act", [torch.bfloat16, torch.float16])
+def test_many_rows(M, N, K, gs, act):
+    """The tiled kernel at the edges of its tiles, slices and stages, weights over all
+    of int8 (-128 among them), x and y in strided rows, with a bias, against float64
+    and, without the workspace of the K slices, against itself in one slice."""
+    if gs > K:
+        gs = 0
+    g = workloads.device_generator(DEV, M + N)
+    w = torch.randint(-128, 128, (N, K), generator=g, device=DEV, dtype=torch.int32).to(torch.int8)
+    shape = (N, K // gs) if gs else (N,)
+    s = (torch.rand(shape, generator=g, device=DEV) * 3e-3 + 1e-3).to(act)
+    x = torch.randn((M, K + 8), generator=g, device=DEV).to(act)[:, 8:]
+    bias = torch.randn((N,), generator=g, device=DEV).to(act)
+    buf = torch.full((M, N + 5), float("nan"), device=DEV).to(act)
+    y = buf[:, :N]
+    lib = _lib.load()
+
+    def call(ws):
+        rc = lib.sd_w8a16_linear(x.data_ptr(), x.stride(0), w.data_ptr(), K, s.data_ptr(),
+                                 _lib.dtype_code(act), gs, bias.data_ptr(), y.data_ptr(),
+                                 y.stride(0), M, N, K, _lib.dtype_code(act),
+                                 None if ws is None else ws.data_ptr(),
+                                 0 if ws is None else ws.numel(), _lib.stream_ptr(x.device))
+        _lib.check(rc)
+        return y.clone()
+
+    nbytes = lib.sd_w8a16_workspace_size(M, N, K, gs)
+    if (M, gs) in ((129, 0), (200, 128)):
+        assert nbytes > 0  # K slices at these sizes
+    got = call(torch.empty(nbytes, dtype=torch.uint8, device=DEV) if nbytes else None)
+    one = call(None)
+    assert torch.equal(got, ops.w8a16_linear(x, w, s, bias, group_size=gs))
+    assert bool(buf[:, N:].isnan().all())
+    rel = 2.0 ** -9 if act == torch.float16 else 2.0 ** -8
+    rows = torch.unique(torch.tensor([0, 1, 15, 16, M // 2, M - 2, M - 1])).to(DEV)
+    for out in (got, one):
+        check(out[rows], x[rows], w, s, bias, "per_group" if gs else "per_channel", gs, out_rel=rel,
+              what=f"{M}x{N}x{K} group {gs}")
+    # every row: the same sums in fp32 (float64 above pins the sampled rows)
+    wf = w.float() * (s.float().repeat_interleave(gs, 1) if gs else s.float()[:, None])
+    ref = x.float() @ wf.T.contiguous() + bias.float()
+    err = (got.float() - ref).abs() - 2 * rel * ref.abs() - 2.0 ** -15 * (x.float().abs() @ wf.abs().T.contiguous())
+    assert float(err.max()) <= 0
+
+
 # ------------------------------------------------- wide matrices at one row
 @pytest.mark.parametrize("N,K", [(151936, 1024), (16411, 2048), (32771, 1024), (8209, 4096)])
 @pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
