@@ -10,22 +10,40 @@
 //
 // Work: one workgroup per (128-row tile, kv head, sequence); the 128 rows are
 // 128 / G consecutive tokens x the G query heads sharing the kv head, heaviest
-// (last) tiles dispatched first. Each of the 4 wave64s owns 32 rows (two
-// 16-row MFMA tiles, so every K / V operand read from LDS feeds two MFMAs)
-// and its own online softmax. Per step of 64 keys the workgroup stages K and
-// V in LDS (double-buffered: one barrier per step; all 256 threads, 16-byte
-// loads, the next step's rows in flight in registers meanwhile) and every wave
-// computes
-//   S^T = K . Q^T      32 x MFMA 16x16x32 (K is the A operand, read from LDS)
+// (last) tiles dispatched first. Each of the 8 wave64s owns 16 rows and its own
+// online softmax. Per step of 64 keys the K and V rows go straight from HBM / L2
+// into LDS (global_load_lds, two stages: the next step's rows land while this step
+// computes, one barrier per step) and every wave computes
+//   S^T = K . Q^T      16 x MFMA 16x16x32 (K is the A operand, read from LDS)
 //   online softmax     exp2 domain, one row per lane (l % 16)
-//   O^T += V^T . P^T   32 x MFMA (P rounded once; 64 with the lo part of P for
-//                      waves with rows that see few keys), V^T gathered with
+//   O^T += V^T . P^T   16 x MFMA (P rounded once; 32 with the lo part of P for
+//                      tiles with rows that see few keys), V^T gathered with
 //                      ds_read_b64_tr_b16
 // Rows are written normalised at the end (no split over keys: a prefill has
 // rows enough to fill the machine).
+//
+// Bound: the issue of the softmax's vector instructions beside the MFMAs, and power
+// (4 x 2048 tokens, 32 heads over 8: 35% MFMA-busy at 2.1 GHz; a clock of 2.4 GHz falls
+// as the kernel gets denser). Four waves per SIMD hide each other's LDS and barrier waits:
+// 8 waves of 16 rows against 4 of 32 (half the LDS reads, two waves per SIMD) measured 184
+// against 181 us there, 114 against 119 on ragged prompts over cached pages. The version
+// that staged rows through registers, rescaled at every rise in any of 32 rows and ran
+// each tile on any XCD took 354 and 268 us.
+// What the loop leaves out:
+//  * the lane exchange and the rescaling of 32 accumulators happen only where a vote says
+//    that a maximum of the wave's 16 rows rises. (Raising it only by more than 1, 2 or 8 in
+//    log2 units measured 3, 5 and 7% faster, but the rows' largest weight is then no longer
+//    exactly 1: 1 - 4% more error against 64 bits.)
+//  * the row sums of P come from the matrix cores too (a row of ones times P^T): 2
+//    MFMAs instead of 16 additions, and the weights that are divided out are the rounded
+//    ones that multiplied V;
+//  * the scale is folded into the exponent's multiply-add; a negative scale flips the
+//    signs of q instead.
+// All tiles of a (sequence, kv head) run on one XCD where the pairs divide by 8, so its
+// K / V rows are read from that XCD's L2 (4 MB; 2048 keys are 1 MB).
 #include <math.h>
 
-#include <algorithm>
+#include <type_traits>
 
 #include "sd_common.h"
 
@@ -35,12 +53,13 @@ using sd::f32x4;
 using sd::u32x4;
 
 constexpr int kD = 128;
-constexpr int kThreads = 256;
-constexpr int kRT = 2;                  // 16-row MFMA tiles per wave
-constexpr int kRows = 4 * 16 * kRT;     // query rows per workgroup (4 waves x 32)
+constexpr int kWaves = 8;
+constexpr int kThreads = 64 * kWaves;
+constexpr int kRT = 1;                    // 16-row MFMA tiles per wave
+constexpr int kRows = kWaves * 16 * kRT;  // query rows per workgroup
 constexpr int kKeys = 64;               // keys per step
-constexpr int kKPitch = 136;   // LDS row pitch of the K tile (16-bit elements)
-constexpr int kVPitch = 144;   // LDS row pitch of the V tile
+constexpr int kRowBytes = kD * 2;            // one key's K (or V) row
+constexpr int kTile = kKeys * kRowBytes;     // one stage: the K tile, then the V tile
 
 struct PrefillParams {
   const uint16_t* q;
@@ -58,65 +77,94 @@ struct PrefillParams {
   const int32_t* cu_k;  // (B + 1,)
   int32_t num_seqs, G, Hkv;
   int64_t total_q;
-  float scale_log2;
+  float scale_log2;   // |scale| log2(e), never 0
+  uint32_t q_flip;    // sign bits of a q pair when the scale is negative
   uint16_t* out;
   int64_t o_stok, o_shead;
+  int32_t by_xcd;  // (head, sequence) pairs are dealt to the XCDs
 };
 
-// Element offset of key `tok` of sequence b (k0 = cu_k[b] for contiguous K/V).
-__device__ __forceinline__ int64_t key_row(const PrefillParams& p, const int32_t* btrow,
-                                           int64_t k0, int tok) {
-  if (!p.bt) return (k0 + tok) * p.s_tok;
-  int pg, off;
-  if (p.bs_shift >= 0) {
-    pg = tok >> p.bs_shift;
-    off = tok & (p.block_size - 1);
-  } else {
-    pg = tok / p.block_size;
-    off = tok - pg * p.block_size;
-  }
-  const int blk = min(max(btrow[pg], 0), p.num_blocks - 1);
-  return static_cast<int64_t>(blk) * p.s_blk + static_cast<int64_t>(off) * p.s_tok;
+// K / V row addressing: contiguous rows; pages that hold whole 64-key steps (one block
+// lookup per page, scalar); anything else (one lookup and a whole address per row).
+enum Rows { kContiguous, kPagedSteps, kAnyRows };
+constexpr int64_t kMaxStep = int64_t{1} << 24;  // row strides below keep a step within 32-bit offsets
+
+// 16 bytes per lane from base + off to LDS byte 16 * lane of the wave-uniform address l.
+// Written as assembly for the scalar-base form (no address arithmetic per step) and because
+// the compiler makes a transpose read of LDS wait for every such load in flight; the loop
+// waits itself, before its barrier. No register is written, and the address registers are
+// read when the instruction issues.
+__device__ __forceinline__ void load_lds16(const char* base, uint32_t off, const void* l) {
+  const uint32_t dst = static_cast<uint32_t>(
+      reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void*)l));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               ::"s"(__builtin_amdgcn_readfirstlane(dst)), "v"(off), "s"(base)
+               : "memory", "m0");
+}
+// The same with a whole address per lane.
+__device__ __forceinline__ void load_lds16(const char* g, const void* l) {
+  const uint32_t dst = static_cast<uint32_t>(
+      reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void*)l));
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               ::"s"(__builtin_amdgcn_readfirstlane(dst)), "v"(g)
+               : "memory", "m0");
 }
 
-// SPLIT: P enters P.V as hi + lo 16-bit parts (~16 mantissa bits, twice the
-// P.V MFMAs), for tiles whose first token sees fewer than kSplitKeys keys:
-// with n keys, rounding each P once costs about 2^-9 |v| / sqrt(n_eff) of
-// absolute error, which nears the 2e-3 output tolerance when only a handful of
-// keys are visible. Other tiles round P once to T, as flash attention does.
-// The host launches both instances over the same grid; each workgroup runs in
-// the one that matches its tile and exits from the other.
+// Tiles whose first token sees fewer than kSplitKeys keys ("split"): P enters P.V
+// as hi + lo 16-bit parts (~16 mantissa bits, twice the P.V MFMAs). With n keys,
+// rounding each P once costs about 2^-9 |v| / sqrt(n_eff) of absolute error, which
+// nears the 2e-3 output tolerance when only a handful of keys are visible. Other
+// tiles round P once to T, as flash attention does. Only the first
+// ceil(kSplitKeys / tokens per tile) tiles of a sequence can be split.
 constexpr int kSplitKeys = 128;
 
-template <typename T, bool SPLIT>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+// Maximum over the four lanes that share l % 16 (v_permlane32_swap / 16_swap of v with
+// itself leave a lane its own and its partner's value).
+__device__ __forceinline__ float max_over_groups(float v) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  v = fmaxf(__builtin_bit_cast(float, static_cast<uint32_t>(a[0])),
+            __builtin_bit_cast(float, static_cast<uint32_t>(a[1])));
+  const uint32_t w = __builtin_bit_cast(uint32_t, v);
+  const auto c = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+  return fmaxf(__builtin_bit_cast(float, static_cast<uint32_t>(c[0])),
+               __builtin_bit_cast(float, static_cast<uint32_t>(c[1])));
+}
+
+template <typename T, Rows ROWS>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4)))
 void prefill_kernel(PrefillParams p) {
-  __shared__ __attribute__((aligned(16))) uint16_t kt[2][kKeys * kKPitch];
-  __shared__ __attribute__((aligned(16))) uint16_t vt[2][kKeys * kVPitch];
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
-  const int h = blockIdx.y, b = blockIdx.z;
+  __shared__ __attribute__((aligned(1024))) char sm[2][2 * kTile];
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // Workgroup -> (tile, kv head, sequence). Consecutive workgroups go to the 8 XCDs in
+  // turn; with a multiple of 8 (head, sequence) pairs each XCD takes every eighth pair,
+  // kPairs of them at a time: the heaviest tile of each, then the next (a heavy tile
+  // started late would run alone at the end), the rows of all of them in that XCD's L2.
+  int tile = static_cast<int>(gridDim.x) - 1 - static_cast<int>(blockIdx.x);
+  int h = blockIdx.y, b = blockIdx.z;
+  if (p.by_xcd) {
+    constexpr uint32_t kPairs = 8;
+    const uint32_t lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    const uint32_t idx = lin >> 3, per = gridDim.y * gridDim.z / 8;
+    const uint32_t chunk = idx / (gridDim.x * kPairs), in = idx - chunk * gridDim.x * kPairs;
+    const uint32_t width = min(kPairs, per - chunk * kPairs);
+    const uint32_t pair = (chunk * kPairs + in % width) * 8 + (lin & 7);
+    tile = static_cast<int>(gridDim.x - 1 - in / width);
+    h = static_cast<int>(pair % gridDim.y);
+    b = static_cast<int>(pair / gridDim.y);
+  }
   const int64_t q0 = p.cu_q[b];
   const int nq = max(p.cu_q[b + 1] - p.cu_q[b], 0);
   const int64_t k0 = p.cu_k[b];
   int nk = max(p.cu_k[b + 1] - p.cu_k[b], 0);
-  if (p.bt) nk = min(nk, p.max_ctx);
+  nk = min(nk, p.max_ctx);
   const int tpw = kRows / p.G;  // tokens per workgroup
-  // SPLIT: the first tiles, in order (a tile's first token sees nk - nq + t0 + 1
-  // keys, so only tiles with t0 < kSplitKeys can need it); otherwise the last
-  // tiles (the most keys under the causal rule) first
-  const int t0 = (SPLIT ? static_cast<int>(blockIdx.x)
-                        : static_cast<int>(gridDim.x) - 1 - static_cast<int>(blockIdx.x)) * tpw;
+  const int t0 = tile * tpw;
   if (t0 >= nq) return;
-  // the split instance covers the first split_tiles tiles; a tile there whose
-  // first token sees fewer than kSplitKeys keys is its, every other tile is
-  // the single-P instance's (also when nk < nq leaves later tiles short of keys)
   const int split_tiles = (kSplitKeys + tpw - 1) / tpw;
-  const bool want_split = t0 < split_tiles * tpw && nk - nq + t0 + 1 < kSplitKeys;
-  if (SPLIT != want_split) return;  // the other instance's tile
+  const bool split = tile < split_tiles && nk - nq + t0 + 1 < kSplitKeys;
   const int tl = min(t0 + tpw, nq) - 1;  // last token of the tile
-  const int32_t* btrow = p.bt ? p.bt + static_cast<int64_t>(b) * p.bt_stride : nullptr;
-  const int64_t hoff = static_cast<int64_t>(h) * p.s_head;
 
   // ---- this lane's rows (one per row tile): Q operand, causal limit
   int lim[kRT], qi[kRT], gq[kRT];
@@ -137,7 +185,7 @@ void prefill_kernel(PrefillParams p) {
         lg * 8;
 #pragma unroll
     for (int s = 0; s < 4; ++s)
-      qop[rt][s] = valid[rt] ? sd::load16(qp + s * 32) : u32x4{0u, 0u, 0u, 0u};
+      qop[rt][s] = valid[rt] ? sd::load16(qp + s * 32) ^ p.q_flip : u32x4{0u, 0u, 0u, 0u};
     wlast = max(wlast, lim[rt]);
     if (valid[rt]) wfull = min(wfull, lim[rt]);
   }
@@ -154,141 +202,192 @@ void prefill_kernel(PrefillParams p) {
   const int glast = nk - nq + tl;
   const int nsteps = glast < 0 ? 0 : (glast + kKeys) / kKeys;
 
-  float m_run[kRT], l_run[kRT];
-  f32x4 acc[kRT][8];
+  float m_run[kRT];
+  f32x4 acc[kRT][8], lsum[kRT];  // lsum: the row's sum of P, in every element
 #pragma unroll
   for (int rt = 0; rt < kRT; ++rt) {
-    m_run[rt] = -INFINITY;
-    l_run[rt] = 0.f;
+    m_run[rt] = -INFINITY;  // the row's largest score (unscaled)
+    lsum[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) acc[rt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
+  const uint32_t one2 = __is_same(T, __bf16) ? 0x3f803f80u : 0x3c003c00u;
+  const u32x4 ones = {one2, one2, one2, one2};
 
-  // ---- K / V staging: thread t loads key (t / 16) + 16 i, dims 8 (t % 16) .. +8
-  const int ld_key = tid >> 4, ld_col = (tid & 15) * 8;
-  constexpr int kLd = kKeys / 16;  // rows per thread per step
-  u32x4 kr[kLd], vr[kLd];
-  auto load = [&](int step) {
-#pragma unroll
-    for (int i = 0; i < kLd; ++i) {
-      const int tok = min(step * kKeys + ld_key + 16 * i, max(nk - 1, 0));
-      const int64_t off = key_row(p, btrow, k0, tok) + hoff + ld_col;
-      kr[i] = sd::load16_stream(p.k + off);
-      vr[i] = sd::load16_stream(p.v + off);
-    }
-  };
-  auto stage = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < kLd; ++i) {
-      sd::store16(kt[buf] + (ld_key + 16 * i) * kKPitch + ld_col, kr[i]);
-      sd::store16(vt[buf] + (ld_key + 16 * i) * kVPitch + ld_col, vr[i]);
-    }
-  };
-  if (nsteps > 0) {
-    load(0);
-    stage(0);
-    if (nsteps > 1) load(1);
-    __syncthreads();
+  // ---- K / V loads: wave w brings rows 16 w .. 16 w + 15 of a step, four 256-byte rows
+  //      per instruction (16 lanes each). The 16-byte unit u of row r lies at position
+  //      u ^ (r & 15) of its K row and u ^ 2 (r & 7) of its V row, so that the K operand
+  //      reads (16 rows, one unit) and the V transpose reads (16 rows, 32 bytes) each
+  //      cover all banks. Rows past the last key read it again (masked).
+  const char* kh = reinterpret_cast<const char*>(p.k + static_cast<int64_t>(h) * p.s_head);
+  const char* vh = reinterpret_cast<const char*>(p.v + static_cast<int64_t>(h) * p.s_head);
+  if (ROWS == kContiguous || !p.bt) {
+    kh += k0 * p.s_tok * 2;
+    vh += k0 * p.s_tok * 2;
   }
-  for (int step = 0; step < nsteps; ++step) {
-    const int buf = step & 1;
-    const uint16_t* kb = kt[buf];
-    const uint16_t* vb = vt[buf];
-    const int tb = step * kKeys;
-    if (tb <= wlast) {  // some row of this wave sees these keys
-      // ---- S^T: lane holds S[row lr][key tb + 16 j + 4 lg + i] per row tile
-      f32x4 sc[kRT][4];
+  const int32_t* btrow = p.bt ? p.bt + static_cast<int64_t>(b) * p.bt_stride : nullptr;
+  // byte offsets of this lane's units from the step's first row (rows of a step lie within
+  // 32 bits of it, but for kAnyRows)
+  const uint32_t row_bytes = static_cast<uint32_t>(p.s_tok) * 2;
+  constexpr int kLd = kKeys / kWaves / 4;  // loads of four rows, K and V each
+  uint32_t koff[kLd], voff[kLd];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        u32x4 ka[4];
+  for (int i = 0; i < kLd; ++i) {
+    const int r = (wave * kLd + i) * 4 + lg;
+    koff[i] = static_cast<uint32_t>(r) * row_bytes + (lr ^ (r & 15)) * 16;
+    voff[i] = static_cast<uint32_t>(r) * row_bytes + (lr ^ ((r & 7) * 2)) * 16;
+  }
+  int page = -1;
+  int64_t page_off = 0;  // bytes
+  auto issue = [&](int step, int st) {
+    char* dst = sm[st] + wave * kLd * 1024;
+    if constexpr (ROWS == kAnyRows) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) ka[s] = sd::load16(kb + (j * 16 + lr) * kKPitch + s * 32 + lg * 8);
-#pragma unroll
-        for (int rt = 0; rt < kRT; ++rt) {
-          f32x4 c = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int s = 0; s < 4; ++s) c = sd::Elem<T>::mfma(ka[s], qop[rt][s], c);
-          sc[rt][j] = c;
+      for (int i = 0; i < kLd; ++i) {
+        const int r = (wave * kLd + i) * 4 + lg, tok = min(step * kKeys + r, nk - 1);
+        int64_t off = static_cast<int64_t>(tok) * p.s_tok * 2;
+        if (btrow) {
+          const int pg = p.bs_shift >= 0 ? tok >> p.bs_shift : tok / p.block_size;
+          const int blk = min(max(btrow[pg], 0), p.num_blocks - 1);
+          off = (static_cast<int64_t>(blk) * p.s_blk + static_cast<int64_t>(tok - pg * p.block_size) * p.s_tok) * 2;
         }
+        load_lds16(kh + off + (lr ^ (r & 15)) * 16, dst + i * 1024);
+        load_lds16(vh + off + (lr ^ ((r & 7) * 2)) * 16, dst + kTile + i * 1024);
       }
-      // ---- online softmax (exp2 domain), P = hi + lo per 32-key half
-      const bool full = tb + kKeys - 1 <= wfull;
-      u32x4 phi[kRT][2], plo[SPLIT ? kRT : 1][2];
+    } else {
+      int64_t first = static_cast<int64_t>(step) * kKeys * p.s_tok * 2;  // the step's first row
+      if constexpr (ROWS == kPagedSteps) {
+        const int pg = step * kKeys / p.block_size;
+        if (pg != page) {  // uniform
+          page = pg;
+          const int blk = min(max(sd::load_scalar_i32(btrow + pg), 0), p.num_blocks - 1);
+          page_off = (static_cast<int64_t>(blk) * p.s_blk - static_cast<int64_t>(pg) * p.block_size * p.s_tok) * 2;
+        }
+        first += page_off;
+      }
+      const int spare = step * kKeys + kKeys - nk;  // rows of the step past the last key
+#pragma unroll
+      for (int i = 0; i < kLd; ++i) {
+        uint32_t ko = koff[i], vo = voff[i];
+        if (spare > 0) {  // (last step)
+          const uint32_t back =
+              static_cast<uint32_t>(max((wave * kLd + i) * 4 + lg - (kKeys - 1 - spare), 0)) * row_bytes;
+          ko -= back;
+          vo -= back;
+        }
+        load_lds16(kh + first, ko, dst + i * 1024);
+        load_lds16(vh + first, vo, dst + kTile + i * 1024);
+      }
+    }
+  };
+  // LDS offsets of this lane's operands. K: row lr (of 16), unit 4 s + lg. V: row
+  // 4 lg + lr / 4, the 8-byte chunk lr % 4 of the 32 bytes of dims 16 dt.
+  const int ka_lane = lr * kRowBytes + ((lg ^ (lr & 3)) * 16);
+  const int va_lane = kTile + (lg * 4 + (lr >> 2)) * kRowBytes +
+                      ((((lg & 1) * 4 + (lr >> 2)) * 32) | ((lr & 3) * 8));
+
+  // one step's math on stage `base`; SPLIT adds the lo part of P
+  auto compute = [&](const char* base, int tb, auto split_tag) {
+    constexpr bool SPLIT = decltype(split_tag)::value;
+    // ---- S^T: lane holds S[row lr][key tb + 16 j + 4 lg + i] per row tile
+    f32x4 sc[kRT][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      u32x4 ka[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        ka[s] = sd::load16(base + (ka_lane | ((s ^ (lr >> 2)) * 64)) + j * 16 * kRowBytes);
 #pragma unroll
       for (int rt = 0; rt < kRT; ++rt) {
-        float mloc = -INFINITY;
+        f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) c = sd::Elem<T>::mfma(ka[s], qop[rt][s], c);
+        sc[rt][j] = c;
+      }
+    }
+    if (tb + kKeys - 1 > wfull) {  // some row of the wave does not see all 64 keys
+#pragma unroll
+      for (int rt = 0; rt < kRT; ++rt)
 #pragma unroll
         for (int j = 0; j < 4; ++j)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            float sv = sc[rt][j][i] * p.scale_log2;
-            if (!full) sv = (tb + j * 16 + lg * 4 + i <= lim[rt]) ? sv : -INFINITY;
-            sc[rt][j][i] = sv;
-            mloc = fmaxf(mloc, sv);
-          }
-        mloc = sd::max_over_groups(mloc);
-        const float mnew = fmaxf(m_run[rt], mloc);
-        const float mb = mnew == -INFINITY ? 0.f : mnew;
-        float ps = 0.f;
+          for (int i = 0; i < 4; ++i)
+            sc[rt][j][i] = tb + j * 16 + lg * 4 + i <= lim[rt] ? sc[rt][j][i] : -INFINITY;
+    }
+    // ---- the rows' maxima; 16 rows are rescaled when one of theirs rises
 #pragma unroll
-        for (int kh = 0; kh < 2; ++kh) {
-          float pv[8];
+    for (int rt = 0; rt < kRT; ++rt) {
+      float m = fmaxf(sc[rt][0][0], sc[rt][0][1]);
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            pv[q] = sd::fast_exp2(sc[rt][2 * kh][q] - mb);
-            pv[4 + q] = sd::fast_exp2(sc[rt][2 * kh + 1][q] - mb);
-          }
+      for (int e = 2; e < 16; e += 2) m = fmaxf(fmaxf(m, sc[rt][e / 4][e % 4]), sc[rt][e / 4][e % 4 + 1]);
+      if (__any(m > m_run[rt])) {
+        const float mnew = fmaxf(m_run[rt], max_over_groups(m));
+        // (m_run = -inf: nothing accumulated yet; both -inf: the row sees no key so far)
+        const float alpha = mnew == -INFINITY ? 1.f : sd::fast_exp2((m_run[rt] - mnew) * p.scale_log2);
+        lsum[rt] *= alpha;
 #pragma unroll
-          for (int q = 0; q < 8; ++q) ps += pv[q];
-          if constexpr (SPLIT) {
-            uint32_t hi[4], lo[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) sd::split_pack<T>(pv[2 * q], pv[2 * q + 1], hi[q], lo[q]);
-            phi[rt][kh] = u32x4{hi[0], hi[1], hi[2], hi[3]};
-            plo[rt][kh] = u32x4{lo[0], lo[1], lo[2], lo[3]};
-          } else {
-            phi[rt][kh] = u32x4{sd::pack2<T>(pv[0], pv[1]), sd::pack2<T>(pv[2], pv[3]),
-                                sd::pack2<T>(pv[4], pv[5]), sd::pack2<T>(pv[6], pv[7])};
-          }
-        }
-        if (__any(mnew > m_run[rt])) {
-          const float alpha = sd::fast_exp2(m_run[rt] - mb);
-          l_run[rt] *= alpha;
-#pragma unroll
-          for (int dt = 0; dt < 8; ++dt) acc[rt][dt] *= alpha;
-        }
-        l_run[rt] += ps;
+        for (int dt = 0; dt < 8; ++dt) acc[rt][dt] *= alpha;
         m_run[rt] = mnew;
       }
-      // ---- O^T += V^T . P^T; in 32-key half kh, k-slot 8 lg + j <-> key
-      //      32 kh + 4 lg + j (j < 4) and 32 kh + 16 + 4 lg + j - 4 (j >= 4)
+    }
+    // ---- P = 2^(scale (s - reference)), per 32-key half
+    u32x4 phi[kRT][2], plo[SPLIT ? kRT : 1][2];
 #pragma unroll
-      for (int kh = 0; kh < 2; ++kh)
+    for (int rt = 0; rt < kRT; ++rt) {
+      const float nb = m_run[rt] == -INFINITY ? 0.f : -m_run[rt] * p.scale_log2;
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt) {
-          const uint16_t* c = vb + (kh * 32 + lg * 4 + (lr >> 2)) * kVPitch + dt * 16 + (lr & 3) * 4;
-          const uint2 v0 = sd::lds_read_tr16(c);
-          const uint2 v1 = sd::lds_read_tr16(c + 16 * kVPitch);
-          const u32x4 vop = {v0.x, v0.y, v1.x, v1.y};
+      for (int kh2 = 0; kh2 < 2; ++kh2) {
+        float pv[8];
 #pragma unroll
-          for (int rt = 0; rt < kRT; ++rt) {
-            acc[rt][dt] = sd::Elem<T>::mfma(vop, phi[rt][kh], acc[rt][dt]);
-            if constexpr (SPLIT) acc[rt][dt] = sd::Elem<T>::mfma(vop, plo[rt][kh], acc[rt][dt]);
-          }
+        for (int q = 0; q < 8; ++q)
+          pv[q] = sd::fast_exp2(__builtin_fmaf(sc[rt][2 * kh2 + q / 4][q % 4], p.scale_log2, nb));
+        if constexpr (SPLIT) {
+          uint32_t hi[4], lo[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) sd::split_pack<T>(pv[2 * q], pv[2 * q + 1], hi[q], lo[q]);
+          phi[rt][kh2] = u32x4{hi[0], hi[1], hi[2], hi[3]};
+          plo[rt][kh2] = u32x4{lo[0], lo[1], lo[2], lo[3]};
+        } else {
+          phi[rt][kh2] = u32x4{sd::pack2<T>(pv[0], pv[1]), sd::pack2<T>(pv[2], pv[3]),
+                               sd::pack2<T>(pv[4], pv[5]), sd::pack2<T>(pv[6], pv[7])};
         }
+        lsum[rt] = sd::Elem<T>::mfma(ones, phi[rt][kh2], lsum[rt]);
+        if constexpr (SPLIT) lsum[rt] = sd::Elem<T>::mfma(ones, plo[rt][kh2], lsum[rt]);
+      }
     }
-    // ---- next step's tile into the other buffer (its readers finished at the
-    //      previous barrier), then the one barrier of this step
-    if (step + 1 < nsteps) {
-      stage(buf ^ 1);
-      if (step + 2 < nsteps) load(step + 2);
+    // ---- O^T += V^T . P^T; in 32-key half kh2, k-slot 8 lg + j <-> key
+    //      32 kh2 + 4 lg + j (j < 4) and 32 kh2 + 16 + 4 lg + j - 4 (j >= 4)
+#pragma unroll
+    for (int kh2 = 0; kh2 < 2; ++kh2)
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt) {
+        const char* c = base + (va_lane ^ (dt * 32)) + kh2 * 32 * kRowBytes;
+        const uint2 v0 = sd::lds_read_tr16(c);
+        const uint2 v1 = sd::lds_read_tr16(c + 16 * kRowBytes);
+        const u32x4 vop = {v0.x, v0.y, v1.x, v1.y};
+#pragma unroll
+        for (int rt = 0; rt < kRT; ++rt) {
+          acc[rt][dt] = sd::Elem<T>::mfma(vop, phi[rt][kh2], acc[rt][dt]);
+          if constexpr (SPLIT) acc[rt][dt] = sd::Elem<T>::mfma(vop, plo[rt][kh2], acc[rt][dt]);
+        }
+      }
+  };
+  auto loop = [&](auto split_tag) {
+    for (int step = 0; step < nsteps; ++step) {
+      // this step's rows have landed, and every wave is done with the other stage
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (step + 1 < nsteps) issue(step + 1, (step + 1) & 1);
+      if (step * kKeys <= wlast) compute(sm[step & 1], step * kKeys, split_tag);
     }
-    __syncthreads();
-  }
+  };
+  if (nsteps > 0) issue(0, 0);
+  if (split) loop(std::true_type{});
+  else loop(std::false_type{});
+
   // ---- normalised rows: lane holds O[row lr][dims 16 dt + 4 lg .. +4]
 #pragma unroll
   for (int rt = 0; rt < kRT; ++rt) {
-    const float l = sd::sum_over_groups(l_run[rt]);
+    const float l = lsum[rt][0];
     if (!valid[rt]) continue;
     const float inv = l > 0.f ? 1.f / l : 0.f;
     uint16_t* op = p.out + (q0 + qi[rt]) * p.o_stok +
@@ -301,6 +400,16 @@ void prefill_kernel(PrefillParams p) {
       *reinterpret_cast<uint2*>(op + dt * 16 + lg * 4) = w;
     }
   }
+}
+
+template <typename T>
+void launch(const PrefillParams& p, dim3 grid, hipStream_t st) {
+  if (!p.bt && p.s_tok < kMaxStep)
+    hipLaunchKernelGGL((prefill_kernel<T, kContiguous>), grid, dim3(kThreads), 0, st, p);
+  else if (p.block_size % kKeys == 0 && p.s_tok < kMaxStep)
+    hipLaunchKernelGGL((prefill_kernel<T, kPagedSteps>), grid, dim3(kThreads), 0, st, p);
+  else
+    hipLaunchKernelGGL((prefill_kernel<T, kAnyRows>), grid, dim3(kThreads), 0, st, p);
 }
 
 }  // namespace
@@ -378,24 +487,20 @@ extern "C" int sd_prefill_attention(
   p.G = G;
   p.Hkv = num_kv_heads;
   p.total_q = total_q;
-  p.scale_log2 = scale * 1.4426950408889634f;
+  const float mag = fabsf(scale) * 1.4426950408889634f;
+  p.scale_log2 = mag == 0.f ? 1e-37f : mag;  // (0 would turn a masked score's -inf into NaN)
+  p.q_flip = scale < 0.f ? 0x80008000u : 0u;
   p.out = static_cast<uint16_t*>(out);
   p.o_stok = out_stride_tok;
   p.o_shead = out_stride_head;
   const int tpw = kRows / G;
-  const dim3 grid(static_cast<unsigned>((max_seqlen_q + tpw - 1) / tpw),
+  const int64_t longest = max_seqlen_q < total_q ? max_seqlen_q : total_q;
+  const dim3 grid(static_cast<unsigned>((longest + tpw - 1) / tpw),
                   static_cast<unsigned>(num_kv_heads), static_cast<unsigned>(num_seqs));
   hipStream_t st = static_cast<hipStream_t>(stream);
-  // the tiles whose rows see few keys (split P; at most the first
-  // ceil(kSplitKeys / tpw) tiles of a sequence), then the rest (P rounded once)
-  const dim3 sgrid(std::min(grid.x, static_cast<unsigned>((kSplitKeys + tpw - 1) / tpw)), grid.y,
-                   grid.z);
-  if (dtype == SD_BF16) {
-    hipLaunchKernelGGL((prefill_kernel<__bf16, true>), sgrid, dim3(kThreads), 0, st, p);
-    hipLaunchKernelGGL((prefill_kernel<__bf16, false>), grid, dim3(kThreads), 0, st, p);
-  } else {
-    hipLaunchKernelGGL((prefill_kernel<_Float16, true>), sgrid, dim3(kThreads), 0, st, p);
-    hipLaunchKernelGGL((prefill_kernel<_Float16, false>), grid, dim3(kThreads), 0, st, p);
-  }
+  const int64_t pairs = static_cast<int64_t>(num_kv_heads) * num_seqs;
+  p.by_xcd = pairs % 8 == 0 && pairs * grid.x < (int64_t{1} << 31);
+  if (dtype == SD_BF16) launch<__bf16>(p, grid, st);
+  else launch<_Float16>(p, grid, st);
   return sd::check_launch("prefill_attention");
 }

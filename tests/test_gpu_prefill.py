@@ -152,3 +152,41 @@ def test_attention_layer_prefill_stores_and_attends():
     assert_close_attn(to_np(o.float()), ref_varlen(q, k, v, cu_q, cu_k, 128 ** -0.5),
                       what="layer prefill")
     assert torch.equal(layer.k_cache[3, :70].cpu(), k[:70]) and torch.equal(layer.v_cache[5, :9].cpu(), v[70:])
+
+
+@pytest.mark.parametrize("scale", [-0.08, 0.0, 0.3])
+def test_scale_signs(scale):
+    # the scale enters the exponent's multiply-add, its sign the bits of q; 0.3 makes rows
+    # that a single key dominates
+    lens = [130, 65]
+    q, k, v, cu_q, cu_k = make(lens, lens, 16, 8, seed=21)
+    o = ops.prefill_attention(q.to(DEV), k.to(DEV), v.to(DEV), cu_q.to(DEV), cu_k.to(DEV),
+                              max(lens), scale)
+    assert_close_attn(to_np(o.float()), ref_varlen(q, k, v, cu_q, cu_k, scale), what=f"scale {scale}")
+
+
+@pytest.mark.parametrize("bs", [64, 48])
+def test_many_pairs_over_pages(bs):
+    # 9 sequences x 8 kv heads: 9 pairs per XCD, one past the 8 that run together; pages
+    # that hold whole 64-key steps, and pages that do not
+    lq = [1, 63, 64, 65, 127, 128, 129, 31, 40]
+    lk = [n + p for n, p in zip(lq, [0, 1, 64, 63, 0, 7, 128, 200, 0])]
+    q, k, v, cu_q, cu_k = make(lq, lk, 16, 8, torch.float16, seed=bs)
+    kc, vc, bt = _paged(k, v, cu_k, bs, seed=bs)
+    o = ops.prefill_attention(q.to(DEV), kc.to(DEV), vc.to(DEV), cu_q.to(DEV), cu_k.to(DEV),
+                              max(lq), 128 ** -0.5, block_table=bt.to(DEV))
+    assert_close_attn(to_np(o.float()), ref_varlen(q, k, v, cu_q, cu_k, 128 ** -0.5),
+                      what=f"many pairs bs={bs}")
+
+
+def test_row_strides_past_the_short_offsets():
+    # a token stride of 2^24 elements: whole addresses per row instead of 32-bit offsets
+    n = 66
+    q, k, v, cu_q, cu_k = make([n], [n], 8, 8, seed=33)
+    buf = torch.empty((2 * n * (1 << 24),), dtype=torch.bfloat16, device=DEV)
+    kd = buf.as_strided((n, 8, 128), (1 << 24, 128, 1), 0)
+    vd = buf.as_strided((n, 8, 128), (1 << 24, 128, 1), n * (1 << 24))
+    kd.copy_(k)
+    vd.copy_(v)
+    o = ops.prefill_attention(q.to(DEV), kd, vd, cu_q.to(DEV), cu_k.to(DEV), n, 128 ** -0.5)
+    assert_close_attn(to_np(o.float()), ref_varlen(q, k, v, cu_q, cu_k, 128 ** -0.5), what="strides")
