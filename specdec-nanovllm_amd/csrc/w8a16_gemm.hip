@@ -9,9 +9,8 @@
 // about 200 rows up, HBM below. Layout of one step (64 columns of K):
 //  * x rows (128 B) and weight rows (64 B) go from HBM / L2 straight into LDS
 //    (global_load_lds, 16 B per lane, no registers); the 16-byte units of a row are
-//    permuted by the global address of each lane (unit u of x row r lies at position
-//    u ^ (r / 2 & 7), of weight row r at u ^ (r / 4 NT & 3)), so that the 16 lanes of
-//    an operand read hit 16 different 16-byte slots of the 256-byte bank row;
+//    permuted by the global address of each lane, so that the 16 lanes of an operand read
+//    hit 16 different 16-byte slots of the 256-byte bank row (x_swizzle, w_swizzle);
 //  * the weights stay int8 in LDS (half the LDS traffic of a 16-bit tile) and each
 //    wave dequantizes the operands it reads (sd::dequant8): 96 VALU instructions beside
 //    64 MFMAs per wave and step at 128 x 64 outputs per wave;
@@ -55,15 +54,27 @@ template <int N> __device__ __forceinline__ void wait_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-// WM x WN waves, each MT x NT tiles of 16 x 16 outputs; S stages of 64 columns.
-template <typename T, int WM, int WN, int MT, int NT, int S, int WPE, bool PG, bool FLOOR>
+// Position of a 16-byte unit within its LDS row: XOR with these. An operand read takes one
+// unit of 16 x rows, or of the weight rows 4 NT j + i (i, j < 4): with two 128-byte x rows
+// (four 64-byte weight rows) to a 256-byte bank row when KB is 1, whole bank rows (two
+// 128-byte ones) when it is 2, the 16 lanes then cover 16 different 16-byte slots.
+template <int KB> __device__ __forceinline__ int x_swizzle(int r) { return KB == 1 ? (r >> 1) & 7 : r & 15; }
+template <int KB, int NT> __device__ __forceinline__ int w_swizzle(int r) {
+  const int j = (r / (4 * NT)) & 3;
+  return KB == 1 ? j : (((r >> 1) & 1) | (j << 1));
+}
+
+// WM x WN waves, each MT x NT tiles of 16 x 16 outputs; S stages of KB 64-column steps.
+template <typename T, int WM, int WN, int MT, int NT, int S, int KB, int WPE, bool PG, bool FLOOR>
 __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
 void w8a16_gemm_kernel(GemmParams p) {
   constexpr int NW = WM * WN, BM = WM * MT * 16, BN = WN * NT * 16;
-  constexpr int XB = BM * 128, SB = XB + BN * 64;  // bytes of a stage: x rows, weight rows
-  constexpr int CX = BM / 8 / NW, CW = BN / 16 / NW;  // 1 KB loads per wave and stage
+  constexpr int XR = 128 * KB, WR = 64 * KB;       // bytes of an x row, of a weight row
+  constexpr int XB = BM * XR, SB = XB + BN * WR;   // bytes of a stage: x rows, weight rows
+  constexpr int CX = XB / 1024 / NW, CW = BN * WR / 1024 / NW;  // 1 KB loads per wave and stage
   constexpr int LPW = CX + CW;
-  static_assert(CX * NW * 8 == BM && CW * NW * 16 == BN && NT % 2 == 0, "whole 1 KB loads per wave");
+  static_assert(CX * NW * 1024 == XB && CW * NW * 1024 == SB - XB, "whole 1 KB loads per wave");
+  static_assert(KB == 1 || (KB == 2 && !PG), "stages of one or two steps");
   extern __shared__ __attribute__((aligned(1024))) char sm[];
   const sd::W8GemmArgs& a = p.a;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -89,24 +100,26 @@ void w8a16_gemm_kernel(GemmParams p) {
   const int ks = static_cast<int>(static_cast<int64_t>(slice) * p.nks / p.splits);
   const int ke = static_cast<int>(static_cast<int64_t>(slice + 1) * p.nks / p.splits);
 
-  // ---- loads: this lane's 16-byte unit of each 1 KB (8 x rows, 16 weight rows); rows
+  // ---- loads: this lane's 16-byte unit of each 1 KB (of whole x or weight rows); rows
   //      past M / N read the last row (their outputs are not written), steps past the
-  //      slice read its last step (into a stage nobody reads)
+  //      slice read its last ones (into a stage nobody reads)
   const char* xbase = reinterpret_cast<const char*>(a.x + static_cast<int64_t>(m0) * a.xs);
   const char* wbase = reinterpret_cast<const char*>(a.w + static_cast<int64_t>(n0) * a.ws);
   uint32_t xoff[CX], woff[CW];
 #pragma unroll
   for (int i = 0; i < CX; ++i) {
-    const int r = (wave * CX + i) * 8 + (lane >> 3), unit = (lane & 7) ^ ((r >> 1) & 7);
+    const int at = (wave * CX + i) * 64 + lane, r = at / (XR / 16);
+    const int unit = (at % (XR / 16)) ^ x_swizzle<KB>(r);
     xoff[i] = static_cast<uint32_t>(min(r, a.M - 1 - m0)) * static_cast<uint32_t>(a.xs * 2) + unit * 16;
   }
 #pragma unroll
   for (int i = 0; i < CW; ++i) {
-    const int r = (wave * CW + i) * 16 + (lane >> 2), unit = (lane & 3) ^ ((r / (4 * NT)) & 3);
+    const int at = (wave * CW + i) * 64 + lane, r = at / (WR / 16);
+    const int unit = (at % (WR / 16)) ^ w_swizzle<KB, NT>(r);
     woff[i] = static_cast<uint32_t>(min(r, a.N - 1 - n0)) * static_cast<uint32_t>(a.ws) + unit * 16;
   }
   auto issue = [&](int step, int st) {
-    const int s = min(step, ke - 1);
+    const int s = min(step, ke - KB);
     const char* xb = xbase + static_cast<int64_t>(s) * 128;
     const char* wb = wbase + static_cast<int64_t>(s) * 64;
     char* stage = sm + st * SB;
@@ -118,12 +131,12 @@ void w8a16_gemm_kernel(GemmParams p) {
 
   if constexpr (FLOOR) {  // the loads and barriers alone
 #pragma unroll
-    for (int s = 0; s < S; ++s) issue(ks + s, s);
+    for (int s = 0; s < S; ++s) issue(ks + s * KB, s);
     wait_barrier<(S - 1) * LPW>();
     int st = 0;
-    for (int step = ks; step < ke; ++step) {
+    for (int step = ks; step < ke; step += KB) {
       wait_barrier<(S - 2) * LPW>();
-      issue(step + S, st);
+      issue(step + S * KB, st);
       st = st + 1 == S ? 0 : st + 1;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -158,20 +171,22 @@ void w8a16_gemm_kernel(GemmParams p) {
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // ---- LDS operand addresses: x row lr of tile m, 16-byte unit 2 lg + half; weight
-  //      row of tile t, unit lg (16 int8: both halves)
-  const int xa = (wm * MT * 16 + lr) * 128 + (((lg * 2) ^ ((lr >> 1) & 7)) * 16);
-  const int wa = XB + (wn * NT * 16 + (lr >> 2) * 4 * NT + (lr & 3)) * 64 + ((lg ^ (lr >> 2)) * 16);
+  // ---- LDS operand addresses. x: row lr of tile m; half h (32 columns) of a stage takes the
+  //      16-byte unit 8 (h / 2) + 2 lg + h % 2. Weights: row 4 NT (lr / 4) + 4 t + lr % 4 of
+  //      the wave, unit 4 (h / 2) + lg (16 int8: two halves).
+  const int xrow = wm * MT * 16 + lr, wrow = wn * NT * 16 + (lr >> 2) * 4 * NT + (lr & 3);
+  const int xa = xrow * XR + ((lg * 2) ^ x_swizzle<KB>(xrow)) * 16;
+  const int wa = XB + wrow * WR + (lg ^ w_swizzle<KB, NT>(wrow)) * 16;
   u32x4 xf[2][MT], wr[NT];
-  auto read_x = [&](int st, int half) {
-    const char* b = sm + st * SB + (xa ^ (half * 16));
+  auto read_x = [&](int st, int h) {
+    const char* b = sm + st * SB + (xa ^ ((h & 1) * 16 + (h >> 1) * 128));
 #pragma unroll
-    for (int m = 0; m < MT; ++m) xf[half][m] = sd::load16(b + m * 2048);
+    for (int m = 0; m < MT; ++m) xf[h & 1][m] = sd::load16(b + m * 16 * XR);
   };
-  auto read_w = [&](int st) {
-    const char* b = sm + st * SB + wa;
+  auto read_w = [&](int st, int step) {
+    const char* b = sm + st * SB + (wa ^ (step * 64));
 #pragma unroll
-    for (int t = 0; t < NT; ++t) wr[t] = sd::load16(b + t * 256);
+    for (int t = 0; t < NT; ++t) wr[t] = sd::load16(b + t * 4 * WR);
   };
 
   int st = 0;
@@ -182,7 +197,7 @@ void w8a16_gemm_kernel(GemmParams p) {
     for (int step = ks; step < ke; ++step) {
       wait_barrier<(S - 2) * LPW>();
       issue(step + S - 1, st == 0 ? S - 1 : st - 1);
-      read_w(st);
+      read_w(st, 0);
       read_x(st, 0);
       read_x(st, 1);
       const float* tg = tab + (step / spg - g0) * BN + (nb - n0);
@@ -205,30 +220,32 @@ void w8a16_gemm_kernel(GemmParams p) {
     }
   } else {
 #pragma unroll
-    for (int s = 0; s < S; ++s) issue(ks + s, s);
+    for (int s = 0; s < S; ++s) issue(ks + s * KB, s);
     wait_barrier<(S - 1) * LPW>();
-    read_w(0);
+    read_w(0, 0);
     read_x(0, 0);
-    for (int step = ks; step < ke; ++step) {
-      u32x4 wd[NT];
-      read_x(st, 1);
+    for (int step = ks; step < ke; step += KB) {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) wd[t] = sd::dequant8<T>(wr[t].x, wr[t].y);
+      for (int h = 0; h < 2 * KB; ++h) {
+        u32x4 wd[NT];
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
+        for (int t = 0; t < NT; ++t)
+          wd[t] = h & 1 ? sd::dequant8<T>(wr[t].z, wr[t].w) : sd::dequant8<T>(wr[t].x, wr[t].y);
+        if (h < 2 * KB - 1) {
+          read_x(st, h + 1);
+          if (h & 1) read_w(st, (h + 1) / 2);
+        } else {
+          wait_barrier<(S - 2) * LPW>();
+          issue(step + S * KB, st);
+          st = st + 1 == S ? 0 : st + 1;
+          read_w(st, 0);
+          read_x(st, 0);
+        }
 #pragma unroll
-        for (int m = 0; m < MT; ++m) acc[t][m] = sd::Elem<T>::mfma(wd[t], xf[0][m], acc[t][m]);
+        for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int t = 0; t < NT; ++t) wd[t] = sd::dequant8<T>(wr[t].z, wr[t].w);
-      wait_barrier<(S - 2) * LPW>();
-      issue(step + S, st);
-      st = st + 1 == S ? 0 : st + 1;
-      read_w(st);
-      read_x(st, 0);
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int m = 0; m < MT; ++m) acc[t][m] = sd::Elem<T>::mfma(wd[t], xf[1][m], acc[t][m]);
+          for (int m = 0; m < MT; ++m) acc[t][m] = sd::Elem<T>::mfma(wd[t], xf[h & 1][m], acc[t][m]);
+      }
     }
   }
   // no load of this workgroup may reach LDS after it has ended
@@ -264,11 +281,19 @@ void w8a16_gemm_kernel(GemmParams p) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) v[t][i] = acc[t][m][i] * (PG ? 1.f : sc[PG ? 0 : t][i]) + bi[t][i];
     if (whole) {
+      uint32_t o[2 * NT];
 #pragma unroll
-      for (int t = 0; t < NT; t += 2)
-        sd::store16(dst + 4 * t, u32x4{sd::pack2<T>(v[t][0], v[t][1]), sd::pack2<T>(v[t][2], v[t][3]),
-                                       sd::pack2<T>(v[t + 1][0], v[t + 1][1]),
-                                       sd::pack2<T>(v[t + 1][2], v[t + 1][3])});
+      for (int t = 0; t < NT; ++t) {
+        o[2 * t] = sd::pack2<T>(v[t][0], v[t][1]);
+        o[2 * t + 1] = sd::pack2<T>(v[t][2], v[t][3]);
+      }
+      if constexpr (NT == 1) {
+        *reinterpret_cast<uint2*>(dst) = make_uint2(o[0], o[1]);
+      } else {
+#pragma unroll
+        for (int t = 0; t < NT; t += 2)
+          sd::store16(dst + 4 * t, u32x4{o[2 * t], o[2 * t + 1], o[2 * t + 2], o[2 * t + 3]});
+      }
     } else {
 #pragma unroll
       for (int t = 0; t < NT; ++t)
@@ -317,12 +342,13 @@ __global__ __launch_bounds__(256) void w8a16_gemm_reduce(GemmParams p) {
 }
 
 // ------------------------------------------------------------------- launches
-enum Tile { kT64x128, kT128x128, kT128x256, kT256x256 };
+enum Tile { kT32x64, kT64x64, kT64x128, kT64x256, kT128x128, kT128x256, kT256x256 };
 
 struct Shape {
-  int bm, bn;
+  int bm, bn, kb;
 };
-constexpr Shape kShapes[] = {{64, 128}, {128, 128}, {128, 256}, {256, 256}};
+constexpr Shape kShapes[] = {{32, 64, 2},   {64, 64, 2},   {64, 128, 1}, {64, 256, 1},
+                             {128, 128, 1}, {128, 256, 1}, {256, 256, 1}};
 
 int64_t tiles_of(Tile t, int64_t M, int64_t N) {
   return ((M + kShapes[t].bm - 1) / kShapes[t].bm) * ((N + kShapes[t].bn - 1) / kShapes[t].bn);
@@ -330,18 +356,35 @@ int64_t tiles_of(Tile t, int64_t M, int64_t N) {
 
 int64_t pitch_of(int64_t N) { return (N + 3) / 4 * 4; }
 
-// What a tile costs, in microseconds per 64-column step, measured at 256 CUs (M 17 - 4096;
+// LDS of the per-group scale table of a K slice.
+size_t table_bytes(Tile t, int64_t K, int32_t group, int splits) {
+  if (!group) return 0;
+  const int64_t nks = K / 64, spg = group / 64, per = (nks + splits - 1) / splits;
+  return static_cast<size_t>(kShapes[t].bn) * static_cast<size_t>((per + spg - 2) / spg + 1) * sizeof(float);
+}
+
+// Per-group tiles: stages, their bytes with the table.
+constexpr int kGroupStages64 = 3, kGroupStages128 = 2;
+size_t group_lds(Tile t, int64_t K, int32_t group, int splits) {
+  const size_t stages = t == kT64x128 ? kGroupStages64 : kGroupStages128;
+  return stages * (kShapes[t].bm * 128 + kShapes[t].bn * 64) + table_bytes(t, K, group, splits);
+}
+
+// What a tile costs, in microseconds per 64-column step, measured at 256 CUs (M 17 - 6896;
 // N x K 1024 x 2048 to 19456 x 2560 and 151936 x 1024): `alone` with at most one workgroup
-// per CU, `full` per workgroup of a CU that always has more (4096 x 19456 x 2560: 520, 409,
-// 388, 361 us with the four tiles). Per group the step sums and scales come on top, and the
-// tiles stop at 64 x 64 outputs per wave.
+// per CU, `full` per workgroup of a CU that always has more. The large tiles win where they
+// fill the chip (4096 x 19456 x 2560: 64 x 128 520, 128 x 128 409, 128 x 256 388, 256 x 256
+// 361 us), the small ones at few rows: 19456 x 2560 at M = 24 64 x 128 20.5, 32 x 64 15.0 us;
+// at M = 56 23.0 and 18.6; at M = 100 64 x 128 28.1, 64 x 256 25.5. Per group the step sums
+// and scales come on top, and the tiles stop at 64 x 64 outputs per wave.
 struct Cost {
   Tile tile;
   double alone, full;
 };
-constexpr Cost kCosts[] = {{kT64x128, 0.44, 0.341}, {kT128x128, 0.63, 0.535},
-                           {kT128x256, 0.95, 1.01}, {kT256x256, 1.38, 1.78}};
-constexpr Cost kCostsGroup[] = {{kT64x128, 0.55, 0.425}, {kT128x128, 1.2, 0.72}};
+constexpr Cost kCosts[] = {{kT32x64, 0.18, 0.118},   {kT64x64, 0.26, 0.19},   {kT64x128, 0.44, 0.36}, 
+                           {kT64x256, 0.50, 0.68},   {kT128x128, 0.63, 0.535}, {kT128x256, 1.0, 1.01},
+                           {kT256x256, 1.43, 1.78}};
+constexpr Cost kCostsGroup[] = {{kT64x128, 0.50, 0.38}, {kT128x128, 1.2, 0.82}};
 
 struct Plan {
   Tile tile;
@@ -352,20 +395,24 @@ struct Plan {
 // the mean and the largest share: workgroups of a CU run together), about three steps to
 // fill and drain a tile, and for several slices the second launch and the partial sums
 // through memory (4.3 TB/s). Checked against the measured best of all tiles and slices at
-// the sizes above: within 10% of it.
+// the sizes above: 3% more time in the mean.
 Plan plan_for(int64_t M, int64_t N, int64_t K, int32_t group) {
   const int64_t nks = K / 64;
   const double cus = sd::device_cus();
   Plan best{kT64x128, 1};
   double best_us = 1e30;
   const Cost* costs = group ? kCostsGroup : kCosts;
-  const int ncosts = group ? 2 : 4;
+  const int ncosts = group ? 2 : 7;
   for (int c = 0; c < ncosts; ++c)
     for (int splits = 1; splits <= 16; splits *= 2) {
       if (splits > 1 && nks < 4 * splits) break;
+      if (nks % (kShapes[costs[c].tile].kb * splits) && kShapes[costs[c].tile].kb > 1) break;  // whole stages
+      double full = costs[c].full;
+      // (a scale table that leaves room for one workgroup per CU)
+      if (group && group_lds(costs[c].tile, K, group, splits) > 80 * 1024) full = costs[c].alone;
       const double n = static_cast<double>(tiles_of(costs[c].tile, M, N)) * splits / cus;
       const double whole = static_cast<double>(static_cast<int64_t>(n)) + (n > static_cast<int64_t>(n) ? 1 : 0);
-      const double shared = n > 1 ? 0.5 * (n + whole) * costs[c].full : n * costs[c].full;
+      const double shared = n > 1 ? 0.5 * (n + whole) * full : n * full;
       const double step = shared > costs[c].alone ? shared : costs[c].alone;
       double us = (static_cast<double>((nks + splits - 1) / splits) + 3) * step;
       if (splits > 1) us += 3.5 + 8.0 * splits * static_cast<double>(M) * static_cast<double>(N) / 4.3e6;
@@ -377,40 +424,39 @@ Plan plan_for(int64_t M, int64_t N, int64_t K, int32_t group) {
   return best;
 }
 
-// LDS of the per-group scale table of a K slice.
-size_t table_bytes(Tile t, int64_t K, int32_t group, int splits) {
-  if (!group) return 0;
-  const int64_t nks = K / 64, spg = group / 64, per = (nks + splits - 1) / splits;
-  return static_cast<size_t>(kShapes[t].bn) * static_cast<size_t>((per + spg - 2) / spg + 1) * sizeof(float);
-}
-
-template <typename T, int WM, int WN, int MT, int NT, int S, int WPE, bool PG, bool FLOOR>
+template <typename T, int WM, int WN, int MT, int NT, int S, int KB, int WPE, bool PG, bool FLOOR>
 int launch(GemmParams p, Tile t, hipStream_t st) {
   constexpr int BM = WM * MT * 16, BN = WN * NT * 16;
   p.tiles_m = (p.a.M + BM - 1) / BM;
   p.tiles_n = (p.a.N + BN - 1) / BN;
-  const size_t lds = static_cast<size_t>(S) * (BM * 128 + BN * 64) +
+  const size_t lds = static_cast<size_t>(S) * (BM * 128 + BN * 64) * KB +
                      table_bytes(t, p.a.K, FLOOR ? 0 : p.a.group, p.splits);
-  hipLaunchKernelGGL((w8a16_gemm_kernel<T, WM, WN, MT, NT, S, WPE, PG, FLOOR>),
+  hipLaunchKernelGGL((w8a16_gemm_kernel<T, WM, WN, MT, NT, S, KB, WPE, PG, FLOOR>),
                      dim3(static_cast<unsigned>(p.tiles_m * p.tiles_n * p.splits)),
                      dim3(WM * WN * 64), lds, st, p);
   return SD_OK;
 }
 
-// Stages: four for the small tile (its loads cover HBM latency with one workgroup per CU:
-// M = 56 of 19456 x 2560 took 23 us with two, 20 with four), two elsewhere (more workgroups
-// per CU measured better than more stages: 128 x 128 at 4096 x 19456 x 2560 398 against 424).
+// Waves per tile: the small tiles are bound by instruction issue (one wave issues a vector
+// instruction every 8 cycles or so), so they take 16 weight rows per wave and several
+// workgroups per CU, and read 128-byte pieces of a row. Two stages where the tiles are many:
+// more workgroups per CU measured better than more stages (128 x 128 at 4096 x 19456 x 2560
+// 398 against 424 us), three or four where loads wait for HBM (64 x 128 at M = 56 of
+// 19456 x 2560 23 us with two, 20 with four, 24 with eight and one workgroup per CU).
 template <typename T, bool PG, bool FLOOR>
 int launch_tile(Tile t, const GemmParams& p, hipStream_t st) {
   if constexpr (PG) {
-    if (t == kT64x128) return launch<T, 1, 4, 4, 2, 3, 2, true, FLOOR>(p, t, st);
-    return launch<T, 2, 2, 4, 4, 2, 2, true, FLOOR>(p, t, st);
+    if (t == kT64x128) return launch<T, 1, 4, 4, 2, kGroupStages64, 1, 2, true, FLOOR>(p, t, st);
+    return launch<T, 2, 2, 4, 4, kGroupStages128, 1, 2, true, FLOOR>(p, t, st);
   } else {
     switch (t) {
-      case kT64x128: return launch<T, 1, 4, 4, 2, 4, 2, false, FLOOR>(p, t, st);
-      case kT128x128: return launch<T, 2, 2, 4, 4, 2, 3, false, FLOOR>(p, t, st);
-      case kT128x256: return launch<T, 2, 4, 4, 4, 2, 4, false, FLOOR>(p, t, st);
-      default: return launch<T, 2, 4, 8, 4, 2, 2, false, FLOOR>(p, t, st);
+      case kT32x64: return launch<T, 1, 4, 2, 1, 3, 2, 4, false, FLOOR>(p, t, st);
+      case kT64x64: return launch<T, 1, 4, 4, 1, 3, 2, 4, false, FLOOR>(p, t, st);
+      case kT64x128: return launch<T, 1, 4, 4, 2, 4, 1, 2, false, FLOOR>(p, t, st);
+      case kT64x256: return launch<T, 1, 8, 4, 2, 3, 1, 4, false, FLOOR>(p, t, st);
+      case kT128x128: return launch<T, 2, 2, 4, 4, 2, 1, 3, false, FLOOR>(p, t, st);
+      case kT128x256: return launch<T, 2, 4, 4, 4, 2, 1, 4, false, FLOOR>(p, t, st);
+      default: return launch<T, 2, 4, 8, 4, 2, 1, 2, false, FLOOR>(p, t, st);
     }
   }
 }
@@ -479,10 +525,8 @@ bool w8a16_gemm_fits(const W8GemmArgs& a, const void* workspace, size_t workspac
   const Tile t = plan_for(a.M, a.N, a.K, a.group).tile;
   if (a.xs >= (int64_t{1} << 23)) return false;
   if (tiles_of(t, a.M, a.N) * *splits > 0x7fffffff) return false;
-  const size_t stages = t == kT64x128 ? 3 : 2;  // (per group; the others have no table)
-  return !a.group || stages * (kShapes[t].bm * 128 + kShapes[t].bn * 64) +
-                             table_bytes(t, a.K, a.group, *splits) <=
-                         static_cast<size_t>(device_lds_per_block());
+  // (one slice instead of the planned ones still has whole stages: nks is a multiple)
+  return !a.group || group_lds(t, a.K, a.group, *splits) <= static_cast<size_t>(device_lds_per_block());
 }
 
 int w8a16_gemm(const W8GemmArgs& a, int splits, void* workspace, hipStream_t st, bool floor) {

@@ -359,9 +359,12 @@ def test_gate_up_silu_entry_refuses_shapes_off_its_paths():
 
 
 # ------------------------------------------------------------- many rows
-@pytest.mark.parametrize("M,N,K,gs", [(17, 9000, 1024, 0),      # 64 x 128 tiles, a ragged last one
-                                      (65, 16400, 640, 0),      # one row into the second tile
-                                      (129, 2560, 4096, 0),     # K slices, added by the second launch
+@pytest.mark.parametrize("M,N,K,gs", [(17, 9001, 1024, 0),      # two-step stages, a ragged last tile
+                                      (33, 20010, 640, 0),      # one row into a second 32-row tile
+                                      (40, 9000, 1088, 0),      # an odd number of steps
+                                      (65, 16400, 640, 0),      # one row into a second 64-row tile
+                                      (100, 19456, 192, 0),     # 64 x 256 tiles
+                                      (129, 1030, 9728, 0),     # K slices, added by the second launch
                                       (200, 1030, 2048, 128),   # the same per group, N % 4 != 0
                                       (300, 6144, 1024, 64),    # one scale per step
                                       (257, 24200, 192, 0),     # three steps
