@@ -9,6 +9,7 @@ or was built for another ABI, every op raises.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 
@@ -186,19 +187,31 @@ def dtype_code(dt: torch.dtype) -> int:
 
 def require_device(*tensors: torch.Tensor) -> torch.device:
     """All tensors on one ROCm device; returns it. CPU tensors are an error (no fallback)."""
-    dev = None
+    first, index = None, -1
     for t in tensors:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise RuntimeError(
                 f"specdec_nanovllm_amd ops run only on a ROCm GPU; got a tensor on {t.device}")
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
-            raise RuntimeError(f"tensors on different devices: {dev} vs {t.device}")
-    return dev
+        if first is None:
+            first, index = t, t.get_device()
+        elif t.get_device() != index:
+            raise RuntimeError(f"tensors on different devices: {first.device} vs {t.device}")
+    return None if first is None else first.device
+
+
+# The wrappers' own time is most of a small call's (a launch through ctypes takes 3 us): the
+# device guard and the stream object cost 3 us of it, against 0.4 us for these two.
+_HERE_ALREADY = contextlib.nullcontext()
+
+
+def on_device(dev: torch.device):
+    """``torch.cuda.device(dev)``, nothing where ``dev`` is the current device."""
+    return _HERE_ALREADY if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
 
 
 def stream_ptr(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
+    """The current stream of ``dev``, as the C ABI takes it."""
+    index = torch.cuda.current_device() if dev.index is None else dev.index
+    return torch._C._cuda_getCurrentRawStream(index)

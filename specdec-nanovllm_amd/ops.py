@@ -55,7 +55,7 @@ def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
         return
     slots = _i32(slot_mapping.reshape(-1))
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = lib.sd_store_kvcache(
             key.data_ptr(), key.stride(0), key.stride(1),
             value.data_ptr(), value.stride(0), value.stride(1),
@@ -188,7 +188,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
         new_rows = (key.data_ptr(), key.stride(0), key.stride(1),
                     value.data_ptr(), value.stride(0), value.stride(1), slots.data_ptr())
     if no_alloc:
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.sd_paged_attention_noalloc(
                 q.data_ptr(), q.stride(0), q.stride(1),
                 k_cache.data_ptr(), v_cache.data_ptr(), sb, sp, sh, num_blocks,
@@ -200,7 +200,7 @@ def paged_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tenso
                 _lib.stream_ptr(dev))
         _lib.check(rc)
         return out
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         # the plan (and so the workspace) depends on the device's compute units
         ws_bytes = lib.sd_paged_attention_workspace_size(
             num_seqs, int(max_seqlen_q), num_q_heads, num_kv_heads, head_dim,
@@ -258,7 +258,7 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if num_seqs <= 0 or total_q == 0:
         return out
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = lib.sd_prefill_attention(q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(),
                                       v.data_ptr(), s_tok, s_head, s_blk, num_blocks, block_size,
                                       _ptr(bt), bt_stride, max_blocks, cuq.data_ptr(),
@@ -287,7 +287,7 @@ def w8a16_linear(x: torch.Tensor, qweight: torch.Tensor, scale: torch.Tensor,
     assert qweight.dtype == torch.int8, f"qweight must be int8, got {qweight.dtype}"
     assert qweight.dim() == 2
     N, K = qweight.shape
-    x2 = x.reshape(-1, x.shape[-1])
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     M = x2.shape[0]
     assert x2.shape[1] == K, f"K mismatch: x {tuple(x2.shape)} vs w {tuple(qweight.shape)}"
     if x2.stride(-1) != 1 or (M > 1 and x2.stride(0) % 8 != 0):
@@ -311,7 +311,7 @@ def w8a16_linear(x: torch.Tensor, qweight: torch.Tensor, scale: torch.Tensor,
     if twin == "floor":
         if group_size:
             raise RuntimeError("w8a16 floor twin: per-channel scales only")
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.sd_w8a16_floor(
                 x2.data_ptr(), x2.stride(0), qw.data_ptr(), qw.stride(0),
                 sc.data_ptr(), _lib.dtype_code(sc.dtype), _ptr(b),
@@ -321,14 +321,14 @@ def w8a16_linear(x: torch.Tensor, qweight: torch.Tensor, scale: torch.Tensor,
         return y.view(*x.shape[:-1], N)
     ws_bytes = lib.sd_w8a16_workspace_size(M, N, K, int(group_size))
     ws = _workspace(ws_bytes, dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = lib.sd_w8a16_linear(
             x2.data_ptr(), x2.stride(0), qw.data_ptr(), qw.stride(0),
             sc.data_ptr(), _lib.dtype_code(sc.dtype), int(group_size), _ptr(b),
             y.data_ptr(), y.stride(0), M, N, K, _lib.dtype_code(x.dtype),
             _ptr(ws), ws_bytes, _lib.stream_ptr(dev))
     _lib.check(rc)
-    return y.view(*x.shape[:-1], N)
+    return y if x.dim() == 2 else y.view(*x.shape[:-1], N)
 
 
 
@@ -368,7 +368,7 @@ def w8a16_silu_linear(gate_up: torch.Tensor, qweight: torch.Tensor, scale: torch
     if M == 0:
         return y.view(*gate_up.shape[:-1], N)
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = lib.sd_w8a16_silu_linear(
             g2.data_ptr(), g2.stride(0), qw.data_ptr(), qw.stride(0),
             sc.data_ptr(), _lib.dtype_code(sc.dtype), int(group_size), _ptr(b),
@@ -443,7 +443,7 @@ def w8a16_rmsnorm_linear(x: torch.Tensor, norm_weight: torch.Tensor, eps: float,
     rc = _lib.SD_ERR_UNSUPPORTED
     if _norm_fused(M, K):
         lib = _lib.load()
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.sd_w8a16_rmsnorm_linear(
                 x2.data_ptr(), x2.stride(0), _ptr(r2), 0 if r2 is None else r2.stride(0),
                 _ptr(ro), 0 if ro is None else ro.stride(0), nw.data_ptr(), float(eps),
@@ -456,7 +456,7 @@ def w8a16_rmsnorm_linear(x: torch.Tensor, norm_weight: torch.Tensor, eps: float,
         h = torch.empty_like(x2)
         rsum = ro if ro is not None or r2 is None else torch.empty_like(r2)
         lib = _lib.load()
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.sd_rmsnorm(x2.data_ptr(), x2.stride(0), _ptr(r2),
                                 0 if r2 is None else r2.stride(0), nw.data_ptr(), h.data_ptr(),
                                 h.stride(0), _ptr(rsum), 0 if rsum is None else rsum.stride(0), M,
@@ -523,14 +523,14 @@ def w8a16_gate_up_silu(x: torch.Tensor, qweight: torch.Tensor, scale: torch.Tens
         # the paired projection on the normalised rows
         xa = torch.empty_like(x2)
         rsum = ro if ro is not None or r2 is None else torch.empty_like(r2)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.sd_rmsnorm(x2.data_ptr(), x2.stride(0), _ptr(r2),
                                 0 if r2 is None else r2.stride(0), nw.data_ptr(), xa.data_ptr(),
                                 xa.stride(0), _ptr(rsum), 0 if rsum is None else rsum.stride(0), M,
                                 K, float(eps), _lib.dtype_code(x.dtype), _lib.stream_ptr(dev))
         _lib.check(rc)
         ra = roa = nwa = None
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = lib.sd_w8a16_gate_up_silu(
             xa.data_ptr(), xa.stride(0), _ptr(ra), 0 if ra is None else ra.stride(0),
             _ptr(roa), 0 if roa is None else roa.stride(0), _ptr(nwa), float(eps),
@@ -566,7 +566,7 @@ def quantize_int8(w: torch.Tensor, group_size: int = 0):
     scale = torch.empty((N, K // G), dtype=torch.bfloat16, device=dev)
     if N:
         lib = _lib.load()
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.sd_quantize_int8(w.data_ptr(), w.stride(0), _lib.dtype_code(w.dtype),
                                       q.data_ptr(), q.stride(0), scale.data_ptr(), N, K,
                                       int(group_size), _lib.stream_ptr(dev))
@@ -577,7 +577,7 @@ def quantize_int8(w: torch.Tensor, group_size: int = 0):
 # --------------------------------------------------------------- draft-step neighbours
 def _rows16(t: torch.Tensor, what: str) -> torch.Tensor:
     """2-D (rows, width) view with a unit last stride and 16-byte aligned rows."""
-    t2 = t.reshape(-1, t.shape[-1])
+    t2 = t if t.dim() == 2 else t.reshape(-1, t.shape[-1])
     if t2.stride(-1) != 1 or t2.data_ptr() % 16 or (t2.shape[0] > 1 and t2.stride(0) % 8):
         t2 = t2.contiguous()
     return t2
@@ -604,16 +604,17 @@ def rmsnorm(x: torch.Tensor, weight: torch.Tensor, eps: float,
     rows = x2.shape[0]
     if rows:
         lib = _lib.load()
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.sd_rmsnorm(x2.data_ptr(), x2.stride(0), _ptr(r2), 0 if r2 is None else r2.stride(0),
                                 w.data_ptr(), o.data_ptr(), o.stride(0), _ptr(ro),
                                 0 if ro is None else ro.stride(0), rows, H, float(eps),
                                 _lib.dtype_code(x.dtype), _lib.stream_ptr(dev))
         _lib.check(rc)
-    o = o.view(x.shape)
+    if x.dim() != 2 or out is not None:
+        o = o.view(x.shape)
     if residual is None:
         return o
-    return o, ro.view(x.shape)
+    return o, ro if x.dim() == 2 else ro.view(x.shape)
 
 
 def qk_norm_rope(q: torch.Tensor, k: torch.Tensor, positions: torch.Tensor,
@@ -657,7 +658,7 @@ def qk_norm_rope(q: torch.Tensor, k: torch.Tensor, positions: torch.Tensor,
         slots = _i32(slot_mapping.reshape(-1)).contiguous()
         assert slots.numel() == T
         _lib.require_device(v, k_cache, v_cache, slots)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.sd_qk_norm_rope_store(
                 q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1),
                 v.data_ptr(), v.stride(0), v.stride(1), T, q.shape[1], k.shape[1], 128,
@@ -667,7 +668,7 @@ def qk_norm_rope(q: torch.Tensor, k: torch.Tensor, positions: torch.Tensor,
                 slots.data_ptr(), _lib.dtype_code(q.dtype), _lib.stream_ptr(dev))
         _lib.check(rc)
         return
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = lib.sd_qk_norm_rope(q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0),
                                  k.stride(1), T, q.shape[1], k.shape[1], 128, _ptr(qw), _ptr(kw),
                                  float(eps), pos.data_ptr(), cs.data_ptr(), cs.stride(0),
@@ -685,12 +686,12 @@ def silu_mul(x: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
         else out.reshape(-1, W // 2)
     if x2.shape[0]:
         lib = _lib.load()
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             rc = lib.sd_silu_mul(x2.data_ptr(), x2.stride(0), o.data_ptr(), o.stride(0),
                                  x2.shape[0], W // 2, _lib.dtype_code(x.dtype),
                                  _lib.stream_ptr(dev))
         _lib.check(rc)
-    return o.view(*x.shape[:-1], W // 2)
+    return o if x.dim() == 2 and out is None else o.view(*x.shape[:-1], W // 2)
 
 
 # Philox (seed, offset) per device for calls that bring no rng_state: seeded
@@ -731,7 +732,7 @@ def sample(logits: torch.Tensor, temperatures: torch.Tensor | None = None,
     assert o.dtype == torch.int64 and o.numel() == rows and o.is_contiguous()
     if rows:
         lib = _lib.load()
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             ws_bytes = lib.sd_sample_workspace_size(rows, V)
             ws = _workspace(ws_bytes, dev)
             rc = lib.sd_sample(logits.data_ptr(), logits.stride(0), _lib.dtype_code(logits.dtype),
@@ -775,7 +776,7 @@ def verify_batch(draft: torch.Tensor, target_logits: torch.Tensor, draft_tokens:
     mask = torch.empty((B, k), dtype=torch.bool, device=dev)
     if B:
         lib = _lib.load()
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             ws_bytes = lib.sd_verify_batch_workspace_size(B, k, V)
             ws = _workspace(ws_bytes, dev)
             rc = lib.sd_verify_batch(draft.data_ptr(), draft.stride(0), draft.stride(1),
@@ -801,7 +802,7 @@ def stream_read(buf: torch.Tensor, sink: torch.Tensor, workgroups: int = 0) -> N
     assert buf.is_contiguous() and sink.dtype == torch.int32 and sink.numel() >= 1
     dev = _lib.require_device(buf, sink)
     nbytes = buf.numel() * buf.element_size() // 16 * 16
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         rc = _lib.load().sd_stream_read(buf.data_ptr(), nbytes, sink.data_ptr(),
                                          int(workgroups), _lib.stream_ptr(dev))
     _lib.check(rc)
