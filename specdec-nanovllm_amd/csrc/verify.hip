@@ -20,7 +20,14 @@
 //                  logits (every workgroup of the sequence; a separate launch
 //                  cost more), then the residual race over its slice of the
 //                  accepted position's rows;
-//   finish_kernel  per sequence: merges the slices' races into the bonus.
+//   finish_kernel  per sequence: merges the slices' races into the bonus (3 us; the
+//                  last race workgroup of a sequence doing it behind a counter cost more:
+//                  its agent-scope release took the race from 10.8 to 19.6 us).
+// Bound: HBM for the statistics, latency for the race (row statistics, then the
+// accepted position's rows). 8 sequences, 6 drafts of 151936 fp32 logits: statistics
+// 14.9 -> 12.6 us with the wave merges on DPP moves instead of six shuffled merges,
+// race 12.4 -> 10.8 with 16 lanes per row in one pass (a wave per row through LDS, each a
+// chain of shuffles, before) and the candidates loaded with the statistics.
 // Noise: Philox4x32-10 keyed by rng_state[0]; u_j uses counter (j, b ^ off_hi,
 // off_lo, 1), u_j = (c0 >> 8) 2^-24 in [0, 1); the bonus noise of element i
 // is word i % 4 of the block with counter (i / 4, b ^ off_hi, off_lo, 2) (one
@@ -113,6 +120,35 @@ __device__ __forceinline__ void merge_ml(float& m, float& l, float m2, float l2)
   if (M == -INFINITY) return;
   l = l * sd::fast_exp2(m - M) + l2 * sd::fast_exp2(m2 - M);
   m = M;
+}
+
+// Maximum over each row of 16 lanes / over the wave, in every lane (rotations and quad
+// permutations inside a row, then v_permlane16_swap / 32_swap of v with itself). Every lane of
+// the rows (of the wave) must be active.
+template <int CTRL> __device__ __forceinline__ float dpp_max(float v) {
+  return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                                               0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false)));
+}
+__device__ __forceinline__ float row_max(float v) {
+  return dpp_max<0xB1>(dpp_max<0x4E>(dpp_max<0x124>(dpp_max<0x128>(v))));
+}
+__device__ __forceinline__ float wave_max(float v) {
+  v = row_max(v);
+  const uint32_t u = __builtin_bit_cast(uint32_t, v);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = fmaxf(__builtin_bit_cast(float, static_cast<uint32_t>(a[0])),
+            __builtin_bit_cast(float, static_cast<uint32_t>(a[1])));
+  const uint32_t w = __builtin_bit_cast(uint32_t, v);
+  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return fmaxf(__builtin_bit_cast(float, static_cast<uint32_t>(b[0])),
+               __builtin_bit_cast(float, static_cast<uint32_t>(b[1])));
+}
+__device__ __forceinline__ float row_sum(float v) {
+  return sd::dpp_add<0xB1>(sd::dpp_add<0x4E>(sd::dpp_add<0x124>(sd::dpp_add<0x128>(v))));
+}
+// l of a lane's (m, l) at the common reference M >= m
+__device__ __forceinline__ float at_max(float m, float l, float M) {
+  return M == -INFINITY ? 0.f : l * sd::fast_exp2(m - M);
 }
 
 // Slice `split` of [0, V): ceil(V / nsplit) elements, rounded up to a multiple
@@ -208,8 +244,9 @@ __global__ __launch_bounds__(kThreads) void stats_kernel(VerifyParams p) {
     row_stats(draft_row<DDT>(p, b, r), v0, v1, s2, p.vec4, want, got, m, l);
   else
     row_stats(target_row<TDT>(p, b, r - p.k), v0, v1, s2, p.vec4, want, got, m, l);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) merge_ml(m, l, __shfl_xor(m, off), __shfl_xor(l, off));
+  const float mw = wave_max(m);
+  l = sd::xor_sum_down<32>(at_max(m, l, mw));
+  m = mw;
   const int wave = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) {
     sm[wave] = m;
@@ -269,30 +306,30 @@ struct Race {
 template <int DDT>
 __device__ int accept(const VerifyParams& p, int b, bool writer, float4& rec) {
   __shared__ float rm[2 * kMaxK + 1], rz[2 * kMaxK + 1];
-  __shared__ float2 parts[kMaxParts];
   __shared__ int acc_s;
   const int rows = 2 * p.k + 1;
   const float s2 = 1.4426950408889634f / temperature(p, b);  // log2(e) / T
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  // ---- row statistics: every (row, slice) partial loaded in one round, then
-  //      one wave per row merges its slices
-  const int nparts = rows * p.nsplit;
-  const float2* st = p.stats + static_cast<int64_t>(b) * nparts;
-  for (int t = threadIdx.x; t < nparts; t += kThreads) {
-    const int r = t / p.nsplit;
-    parts[t] = (p.point_mass && r < p.k) ? make_float2(-INFINITY, 0.f) : st[t];
-  }
-  __syncthreads();
-  for (int r = wave; r < rows; r += kThreads / 64) {
+  // the candidates' tokens and recorded logits load with the statistics (lanes past the
+  // candidates read the last one's)
+  const int jc = min(lane, p.k - 1);
+  const float* g = p.gath + static_cast<int64_t>(b) * 2 * p.k;
+  const int64_t x = p.tokens[b * p.tok_sb + jc];
+  const float gd = g[jc], gt = g[p.k + jc];
+  // ---- row statistics: 16 lanes per row merge its slices
+  const float2* st = p.stats + static_cast<int64_t>(b) * rows * p.nsplit;
+  for (int r = threadIdx.x >> 4; r < rows; r += kThreads / 16) {
     float m = -INFINITY, l = 0.f;
-    for (int s = lane; s < p.nsplit; s += 64) {
-      const float2 ps = parts[r * p.nsplit + s];
-      merge_ml(m, l, ps.x, ps.y);
+    if (!(p.point_mass && r < p.k)) {
+      for (int s = threadIdx.x & 15; s < p.nsplit; s += 16) {
+        const float2 ps = st[r * p.nsplit + s];
+        merge_ml(m, l, ps.x, ps.y);
+      }
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) merge_ml(m, l, __shfl_xor(m, off), __shfl_xor(l, off));
-    if (lane == 0) {
-      rm[r] = m;
+    const float M = row_max(m);
+    l = row_sum(at_max(m, l, M));
+    if ((threadIdx.x & 15) == 0) {
+      rm[r] = M;
       rz[r] = l;
     }
   }
@@ -303,14 +340,12 @@ __device__ int accept(const VerifyParams& p, int b, bool writer, float4& rec) {
     bool ok = true;
     const int j = lane;
     if (j < p.k) {
-      const int64_t x = p.tokens[b * p.tok_sb + j];
       float q = 0.f, pt = 0.f;
       if (x >= 0 && x < p.V) {
-        const float* g = p.gath + static_cast<int64_t>(b) * 2 * p.k;
         // point-mass drafts skip the statistics pass: their value is read here
-        const float dv = p.point_mass ? draft_row<DDT>(p, b, j).at(x) : g[j];
+        const float dv = p.point_mass ? draft_row<DDT>(p, b, j).at(x) : gd;
         q = p.point_mass ? dv : sd::fast_exp2(dv * s2 - rm[j]) / rz[j];
-        pt = sd::fast_exp2(g[p.k + j] * s2 - rm[p.k + j]) / rz[p.k + j];
+        pt = sd::fast_exp2(gt * s2 - rm[p.k + j]) / rz[p.k + j];
       }
       const float ratio = q > 0.f ? fminf(pt / fmaxf(q, 1e-10f), 1.f) : 0.f;
       uint32_t c[4];
