@@ -236,3 +236,39 @@ def test_reference_named_modules():
                              pos.cpu().numpy(), rope.cos_sin_cache.view(4096, 128).cpu().numpy())
     assert_units(to_np(q2.float()).reshape(4, 16, 128), rq, "rope q", units=4, per_row=True)
     assert_units(to_np(k2.float()).reshape(4, 8, 128), rk, "rope k", units=4, per_row=True)
+
+
+@pytest.mark.parametrize("act", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,Hq,Hkv,store,norm,shift", [(128, 16, 8, True, True, 0),   # 3072 heads: the first
+                                                       (131, 32, 8, False, True, 0),  # a partial last workgroup
+                                                       (193, 16, 1, True, False, 0),
+                                                       (200, 16, 8, True, True, 2)])  # rows not 8-byte aligned
+def test_qk_norm_rope_many_heads_same_bits(T, Hq, Hkv, store, norm, shift, act):
+    # four heads per wave from 3072 heads up: bit for bit the one-head-per-wave form, which
+    # runs on the tokens taken 50 at a time; positions past the table, slots of -1 and past
+    # the pool among them
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T + Hq)
+    n = (Hq + 2 * Hkv) * 128
+    buf = torch.randn((T, n + 8), generator=g, device="cuda").to(act)
+    pos = torch.randint(0, 90, (T,), generator=g, device="cuda")
+    cs = torch.randn((80, 128), generator=g, device="cuda")
+    slots = torch.randperm(2 * 256, generator=g, device="cuda")[:T].to(torch.int32)
+    slots[::7] = -1
+    slots[3] = 5000
+    w = [(1 + 0.1 * torch.randn((128,), generator=g, device="cuda")).to(act) if norm else None
+         for _ in range(2)]
+
+    def run(step):
+        x = buf.clone()[:, shift:shift + n]
+        q, k, v = (t.unflatten(-1, (-1, 128)) for t in
+                   x.split([Hq * 128, Hkv * 128, Hkv * 128], dim=-1))
+        kc = torch.zeros((2, 256, Hkv, 128), device="cuda", dtype=act)
+        vc = torch.zeros_like(kc)
+        for a in range(0, T, step):
+            kw = dict(v=v[a:a + step], k_cache=kc, v_cache=vc, slot_mapping=slots[a:a + step]) if store else {}
+            ops.qk_norm_rope(q[a:a + step], k[a:a + step], pos[a:a + step], cs, w[0], w[1], 1e-6, **kw)
+        return x.clone(), kc, vc
+
+    for one, many in zip(run(T), run(50)):
+        assert torch.equal(one.view(torch.int16), many.view(torch.int16))
