@@ -71,9 +71,11 @@ void w8a16_gemm_kernel(GemmParams p) {
   constexpr int NW = WM * WN, BM = WM * MT * 16, BN = WN * NT * 16;
   constexpr int XR = 128 * KB, WR = 64 * KB;       // bytes of an x row, of a weight row
   constexpr int XB = BM * XR, SB = XB + BN * WR;   // bytes of a stage: x rows, weight rows
-  constexpr int CX = XB / 1024 / NW, CW = BN * WR / 1024 / NW;  // 1 KB loads per wave and stage
+  // 1 KB loads per wave and stage: where the x rows don't divide by the waves, the last
+  // waves load the last KB again (the same bytes to the same place, each wave waits for its own)
+  constexpr int KX = XB / 1024, CX = (KX + NW - 1) / NW, CW = BN * WR / 1024 / NW;
   constexpr int LPW = CX + CW;
-  static_assert(CX * NW * 1024 == XB && CW * NW * 1024 == SB - XB, "whole 1 KB loads per wave");
+  static_assert(KX * 1024 == XB && CW * NW * 1024 == SB - XB, "whole 1 KB loads");
   static_assert(KB == 1 || (KB == 2 && !PG), "stages of one or two steps");
   extern __shared__ __attribute__((aligned(1024))) char sm[];
   const sd::W8GemmArgs& a = p.a;
@@ -97,8 +99,9 @@ void w8a16_gemm_kernel(GemmParams p) {
   const int gi = id / (kGroupM * p.tiles_n), gr = id - gi * kGroupM * p.tiles_n;
   const int gm = min(kGroupM, p.tiles_m - gi * kGroupM);
   const int m0 = (gi * kGroupM + gr % gm) * BM, n0 = gr / gm * BN;
-  const int ks = static_cast<int>(static_cast<int64_t>(slice) * p.nks / p.splits);
-  const int ke = static_cast<int>(static_cast<int64_t>(slice + 1) * p.nks / p.splits);
+  const int stages = p.nks / KB;
+  const int ks = KB * static_cast<int>(static_cast<int64_t>(slice) * stages / p.splits);
+  const int ke = KB * static_cast<int>(static_cast<int64_t>(slice + 1) * stages / p.splits);
 
   // ---- loads: this lane's 16-byte unit of each 1 KB (of whole x or weight rows); rows
   //      past M / N read the last row (their outputs are not written), steps past the
@@ -108,7 +111,7 @@ void w8a16_gemm_kernel(GemmParams p) {
   uint32_t xoff[CX], woff[CW];
 #pragma unroll
   for (int i = 0; i < CX; ++i) {
-    const int at = (wave * CX + i) * 64 + lane, r = at / (XR / 16);
+    const int at = min(wave * CX + i, KX - 1) * 64 + lane, r = at / (XR / 16);
     const int unit = (at % (XR / 16)) ^ x_swizzle<KB>(r);
     xoff[i] = static_cast<uint32_t>(min(r, a.M - 1 - m0)) * static_cast<uint32_t>(a.xs * 2) + unit * 16;
   }
@@ -124,7 +127,7 @@ void w8a16_gemm_kernel(GemmParams p) {
     const char* wb = wbase + static_cast<int64_t>(s) * 64;
     char* stage = sm + st * SB;
 #pragma unroll
-    for (int i = 0; i < CX; ++i) load_lds16(xb + xoff[i], stage + (wave * CX + i) * 1024);
+    for (int i = 0; i < CX; ++i) load_lds16(xb + xoff[i], stage + min(wave * CX + i, KX - 1) * 1024);
 #pragma unroll
     for (int i = 0; i < CW; ++i) load_lds16(wb + woff[i], stage + XB + (wave * CW + i) * 1024);
   };
@@ -342,13 +345,13 @@ __global__ __launch_bounds__(256) void w8a16_gemm_reduce(GemmParams p) {
 }
 
 // ------------------------------------------------------------------- launches
-enum Tile { kT32x64, kT64x64, kT64x128, kT64x256, kT128x128, kT128x256, kT256x256 };
+enum Tile { kT32x64, kT64x64, kT64x80, kT64x96, kT64x128, kT64x256, kT128x128, kT128x256, kT256x256 };
 
 struct Shape {
   int bm, bn, kb;
 };
-constexpr Shape kShapes[] = {{32, 64, 2},   {64, 64, 2},   {64, 128, 1}, {64, 256, 1},
-                             {128, 128, 1}, {128, 256, 1}, {256, 256, 1}};
+constexpr Shape kShapes[] = {{32, 64, 2},   {64, 64, 2},   {64, 80, 2},   {64, 96, 2},  {64, 128, 1},
+                             {64, 256, 1},  {128, 128, 1}, {128, 256, 1}, {256, 256, 1}};
 
 int64_t tiles_of(Tile t, int64_t M, int64_t N) {
   return ((M + kShapes[t].bm - 1) / kShapes[t].bm) * ((N + kShapes[t].bn - 1) / kShapes[t].bn);
@@ -375,17 +378,24 @@ size_t group_lds(Tile t, int64_t K, int32_t group, int splits) {
 // per CU, `full` per workgroup of a CU that always has more. The large tiles win where they
 // fill the chip (4096 x 19456 x 2560: 64 x 128 520, 128 x 128 409, 128 x 256 388, 256 x 256
 // 361 us), the small ones at few rows: 19456 x 2560 at M = 24 64 x 128 20.5, 32 x 64 15.0 us;
-// at M = 56 23.0 and 18.6; at M = 100 64 x 128 28.1, 64 x 256 25.5. Per group the step sums
+// at M = 56 23.0 and 18.6; at M = 100 64 x 128 28.1, 64 x 256 25.5). The 80- and 96-row tiles
+// are for widths whose 64-row tiles just miss a whole number of workgroups per CU: 19456 x 2560
+// is 304 tiles of 64 rows, 203 of 96 (weights from HBM: M = 56 21.7 -> 18.6 us, M = 100 64 x 256
+// 29.9, 64 x 80 25.0); five stages instead of three measured 2 - 5% slower there. Per group the step sums
 // and scales come on top, and the tiles stop at 64 x 64 outputs per wave.
 struct Cost {
   Tile tile;
   double alone, full;
 };
-constexpr Cost kCosts[] = {{kT32x64, 0.18, 0.118},   {kT64x64, 0.26, 0.19},   {kT64x128, 0.44, 0.36}, 
-                           {kT64x256, 0.50, 0.68},   {kT128x128, 0.63, 0.535}, {kT128x256, 1.0, 1.01},
-                           {kT256x256, 1.43, 1.78}};
+constexpr Cost kCosts[] = {{kT32x64, 0.188, 0.126},  {kT64x64, 0.256, 0.197},  {kT64x80, 0.307, 0.23},
+                           {kT64x96, 0.303, 0.30},  {kT64x128, 0.44, 0.36},   {kT64x256, 0.50, 0.68},
+                           {kT128x128, 0.63, 0.535}, {kT128x256, 1.0, 1.01},   {kT256x256, 1.43, 1.78}};
 constexpr Cost kCostsGroup[] = {{kT64x128, 0.50, 0.38}, {kT128x128, 1.2, 0.82}};
 
+constexpr int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
+
+// 3, 6 and 12 beside the powers of two: 40 tiles of 2560 rows are 240 workgroups in 6 slices
+// (2560 x 9728, M = 56: 4 slices 18.3 us, 6 slices 15.8; M = 2048 142 -> 114 us with 3).
 struct Plan {
   Tile tile;
   int splits;
@@ -402,11 +412,12 @@ Plan plan_for(int64_t M, int64_t N, int64_t K, int32_t group) {
   Plan best{kT64x128, 1};
   double best_us = 1e30;
   const Cost* costs = group ? kCostsGroup : kCosts;
-  const int ncosts = group ? 2 : 7;
+  const int ncosts = group ? 2 : 9;
   for (int c = 0; c < ncosts; ++c)
-    for (int splits = 1; splits <= 16; splits *= 2) {
+    for (int splits : kSplits) {
+      const int64_t kb = kShapes[costs[c].tile].kb;
       if (splits > 1 && nks < 4 * splits) break;
-      if (nks % (kShapes[costs[c].tile].kb * splits) && kShapes[costs[c].tile].kb > 1) break;  // whole stages
+      if (nks % kb) break;  // whole stages
       double full = costs[c].full;
       // (a scale table that leaves room for one workgroup per CU)
       if (group && group_lds(costs[c].tile, K, group, splits) > 80 * 1024) full = costs[c].alone;
@@ -414,7 +425,7 @@ Plan plan_for(int64_t M, int64_t N, int64_t K, int32_t group) {
       const double whole = static_cast<double>(static_cast<int64_t>(n)) + (n > static_cast<int64_t>(n) ? 1 : 0);
       const double shared = n > 1 ? 0.5 * (n + whole) * full : n * full;
       const double step = shared > costs[c].alone ? shared : costs[c].alone;
-      double us = (static_cast<double>((nks + splits - 1) / splits) + 3) * step;
+      double us = (static_cast<double>((nks / kb + splits - 1) / splits * kb) + 3) * step;
       if (splits > 1) us += 3.5 + 8.0 * splits * static_cast<double>(M) * static_cast<double>(N) / 4.3e6;
       if (us < best_us) {
         best_us = us;
@@ -451,6 +462,8 @@ int launch_tile(Tile t, const GemmParams& p, hipStream_t st) {
   } else {
     switch (t) {
       case kT32x64: return launch<T, 1, 4, 2, 1, 3, 2, 4, false, FLOOR>(p, t, st);
+      case kT64x80: return launch<T, 1, 5, 4, 1, 3, 2, 4, false, FLOOR>(p, t, st);
+      case kT64x96: return launch<T, 1, 6, 4, 1, 3, 2, 4, false, FLOOR>(p, t, st);
       case kT64x64: return launch<T, 1, 4, 4, 1, 3, 2, 4, false, FLOOR>(p, t, st);
       case kT64x128: return launch<T, 1, 4, 4, 2, 4, 1, 2, false, FLOOR>(p, t, st);
       case kT64x256: return launch<T, 1, 8, 4, 2, 3, 1, 4, false, FLOOR>(p, t, st);
@@ -467,8 +480,11 @@ void launch_reduce(const GemmParams& p, hipStream_t st) {
   const dim3 grid(static_cast<unsigned>((n + 255) / 256)), block(256);
   switch (p.splits) {
     case 2: hipLaunchKernelGGL((w8a16_gemm_reduce<T, 2>), grid, block, 0, st, p); break;
+    case 3: hipLaunchKernelGGL((w8a16_gemm_reduce<T, 3>), grid, block, 0, st, p); break;
     case 4: hipLaunchKernelGGL((w8a16_gemm_reduce<T, 4>), grid, block, 0, st, p); break;
+    case 6: hipLaunchKernelGGL((w8a16_gemm_reduce<T, 6>), grid, block, 0, st, p); break;
     case 8: hipLaunchKernelGGL((w8a16_gemm_reduce<T, 8>), grid, block, 0, st, p); break;
+    case 12: hipLaunchKernelGGL((w8a16_gemm_reduce<T, 12>), grid, block, 0, st, p); break;
     default: hipLaunchKernelGGL((w8a16_gemm_reduce<T, 16>), grid, block, 0, st, p); break;
   }
 }

@@ -363,7 +363,10 @@ def test_gate_up_silu_entry_refuses_shapes_off_its_paths():
                                       (33, 20010, 640, 0),      # one row into a second 32-row tile
                                       (40, 9000, 1088, 0),      # an odd number of steps
                                       (65, 16400, 640, 0),      # one row into a second 64-row tile
-                                      (100, 19456, 192, 0),     # 64 x 256 tiles
+                                      (63, 19427, 640, 0),      # 64 x 96 tiles: waves that load the last KB twice
+                                      (100, 19456, 192, 0),     # 64 x 80 tiles
+                                      (125, 19421, 640, 0),     # the same, ragged
+                                      (18, 2570, 9728, 0),      # 12 K slices, a remainder in each
                                       (129, 1030, 9728, 0),     # K slices, added by the second launch
                                       (200, 1030, 2048, 128),   # the same per group, N % 4 != 0
                                       (300, 6144, 1024, 64),    # one scale per step
