@@ -299,7 +299,8 @@ size_t sd_w8a16_workspace_size(int64_t M, int64_t N, int64_t K, int32_t group_si
  * (the lm_head), with batches of 4 rows dealt to the waves in turn; other
  * shapes run the 16-row MFMA kernel (the SiLU and RMSNorm forms below follow the
  * same rule), and past 16 rows most run a tiled MFMA kernel (small layers at
- * up to 128 rows stay on the former). Supported: K % 64 == 0,
+ * up to 128 rows, and more than 32 Mi weights of K <= 1024 at up to 32 rows, stay on
+ * the former). Supported: K % 64 == 0,
  * group_size 0 or a multiple of 64 dividing K; N < 2^24 rows, a row stride
  * below 2^24 bytes and N * w_stride_n < 2^32 bytes (the MFMA kernel forms a
  * row's byte offset with one 24 x 24-bit multiply-add; SD_ERR_UNSUPPORTED

@@ -518,8 +518,12 @@ namespace sd {
 // 1024 x 2048 at M = 56 6.1 us there against 9.2 here, at M = 128 10.0 against 10.5, at
 // M = 256 16.8 against 12.3; 6144 x 1024 at M = 56 9.2 against 11.0, at M = 128 13.6
 // against 12.0). Per group the same line; 2560 x 9728 at M = 17 is 20 us there, 14 here.
+// And except the vocabulary head at up to 32 rows (K <= 1024, more than 32 Mi weights), which
+// the 16-row kernel reads as whole rows, once per block of up to 32 staged rows: 39.4 us there,
+// 43.9 here (norm included, 151936 x 1024); at M = 56 55.4 there, 49.4 here.
 int w8a16_gemm_splits(int64_t M, int64_t N, int64_t K, int32_t group) {
   if (M <= 16) return 0;
+  if (M <= 32 && K <= 1024 && group == 0 && N * K > (int64_t{32} << 20)) return 0;
   if (M <= 128 && N * K <= (int64_t{8} << 20) && static_cast<double>(M) * N * K <= 5.4e8) return 0;
   return plan_for(M, N, K, group).splits;
 }
