@@ -23,25 +23,24 @@
 // rows enough to fill the machine).
 //
 // Bound: the issue of the softmax's vector instructions beside the MFMAs, and power
-// (4 x 2048 tokens, 32 heads over 8: 35% MFMA-busy at 2.1 GHz; a clock of 2.4 GHz falls
-// as the kernel gets denser). Four waves per SIMD hide each other's LDS and barrier waits:
-// 8 waves of 16 rows against 4 of 32 (half the LDS reads, two waves per SIMD) measured 184
-// against 181 us there, 114 against 119 on ragged prompts over cached pages. The version
-// that staged rows through registers, rescaled at every rise in any of 32 rows and ran
-// each tile on any XCD took 354 and 268 us.
+// (a clock of 2.4 GHz falls as the kernel gets denser). 4 x 2048 tokens, 32 heads over 8:
+// 193 us; ragged prompts over cached pages: 117. Four waves per SIMD hide each other's LDS
+// and barrier waits: 8 waves of 16 rows against 4 of 32 (half the LDS reads, two waves per
+// SIMD) measured 184 against 181 us there, 114 against 119, before the row sums went back
+// to fp32 weights. The version that staged rows through registers, rescaled at every rise in
+// any of 32 rows and ran each tile on any XCD took 354 and 266 us, with the same bits.
 // What the loop leaves out:
 //  * the lane exchange and the rescaling of 32 accumulators happen only where a vote says
 //    that a maximum of the wave's 16 rows rises. (Raising it only by more than 1, 2 or 8 in
 //    log2 units measured 3, 5 and 7% faster, but the rows' largest weight is then no longer
 //    exactly 1: 1 - 4% more error against 64 bits.)
-//  * the row sums of P come from the matrix cores too (a row of ones times P^T): 2
-//    MFMAs instead of 16 additions, and the weights that are divided out are the rounded
-//    ones that multiplied V;
-//  * the scale is folded into the exponent's multiply-add; a negative scale flips the
-//    signs of q instead.
+// What it does not leave out (193 and 117 us instead of 184 and 113): the weights enter the
+// row sums in fp32, before they are rounded for P.V (sums of the rounded ones, a row of ones
+// times P^T on the matrix cores, lose in fp16 every weight below 2^-25 of the row's largest),
+// and a score is scaled and rounded once, ahead of the maximum (a multiply-add in the
+// exponent gives other bits).
 // All tiles of a (sequence, kv head) run on one XCD where the pairs divide by 8, so its
 // K / V rows are read from that XCD's L2 (4 MB; 2048 keys are 1 MB).
-#include <math.h>
 
 #include <type_traits>
 
@@ -77,8 +76,7 @@ struct PrefillParams {
   const int32_t* cu_k;  // (B + 1,)
   int32_t num_seqs, G, Hkv;
   int64_t total_q;
-  float scale_log2;   // |scale| log2(e), never 0
-  uint32_t q_flip;    // sign bits of a q pair when the scale is negative
+  float scale_log2;   // scale log2(e)
   uint16_t* out;
   int64_t o_stok, o_shead;
   int32_t by_xcd;  // (head, sequence) pairs are dealt to the XCDs
@@ -185,7 +183,7 @@ void prefill_kernel(PrefillParams p) {
         lg * 8;
 #pragma unroll
     for (int s = 0; s < 4; ++s)
-      qop[rt][s] = valid[rt] ? sd::load16(qp + s * 32) ^ p.q_flip : u32x4{0u, 0u, 0u, 0u};
+      qop[rt][s] = valid[rt] ? sd::load16(qp + s * 32) : u32x4{0u, 0u, 0u, 0u};
     wlast = max(wlast, lim[rt]);
     if (valid[rt]) wfull = min(wfull, lim[rt]);
   }
@@ -202,17 +200,15 @@ void prefill_kernel(PrefillParams p) {
   const int glast = nk - nq + tl;
   const int nsteps = glast < 0 ? 0 : (glast + kKeys) / kKeys;
 
-  float m_run[kRT];
-  f32x4 acc[kRT][8], lsum[kRT];  // lsum: the row's sum of P, in every element
+  float m_run[kRT], l_run[kRT];  // the row's maximum (log2 units); this lane's share of its sum
+  f32x4 acc[kRT][8];
 #pragma unroll
   for (int rt = 0; rt < kRT; ++rt) {
-    m_run[rt] = -INFINITY;  // the row's largest score (unscaled)
-    lsum[rt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    m_run[rt] = -INFINITY;
+    l_run[rt] = 0.f;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) acc[rt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  const uint32_t one2 = __is_same(T, __bf16) ? 0x3f803f80u : 0x3c003c00u;
-  const u32x4 ones = {one2, one2, one2, one2};
 
   // ---- K / V loads: wave w brings rows 16 w .. 16 w + 15 of a step, four 256-byte rows
   //      per instruction (16 lanes each). The 16-byte unit u of row r lies at position
@@ -288,8 +284,9 @@ void prefill_kernel(PrefillParams p) {
 
   // one step's math on stage `base`; SPLIT adds the lo part of P
   auto compute = [&](const char* base, int tb, auto split_tag) {
+#pragma clang fp contract(off)
     constexpr bool SPLIT = decltype(split_tag)::value;
-    // ---- S^T: lane holds S[row lr][key tb + 16 j + 4 lg + i] per row tile
+    // ---- S^T in log2 units: lane holds S[row lr][key tb + 16 j + 4 lg + i] per row tile
     f32x4 sc[kRT][4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -302,7 +299,7 @@ void prefill_kernel(PrefillParams p) {
         f32x4 c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s = 0; s < 4; ++s) c = sd::Elem<T>::mfma(ka[s], qop[rt][s], c);
-        sc[rt][j] = c;
+        sc[rt][j] = c * p.scale_log2;
       }
     }
     if (tb + kKeys - 1 > wfull) {  // some row of the wave does not see all 64 keys
@@ -323,24 +320,27 @@ void prefill_kernel(PrefillParams p) {
       if (__any(m > m_run[rt])) {
         const float mnew = fmaxf(m_run[rt], max_over_groups(m));
         // (m_run = -inf: nothing accumulated yet; both -inf: the row sees no key so far)
-        const float alpha = mnew == -INFINITY ? 1.f : sd::fast_exp2((m_run[rt] - mnew) * p.scale_log2);
-        lsum[rt] *= alpha;
+        const float alpha = mnew == -INFINITY ? 1.f : sd::fast_exp2(m_run[rt] - mnew);
+        l_run[rt] *= alpha;
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) acc[rt][dt] *= alpha;
         m_run[rt] = mnew;
       }
     }
-    // ---- P = 2^(scale (s - reference)), per 32-key half
+    // ---- P = 2^(s - maximum) per 32-key half, summed in fp32 before the rounding
     u32x4 phi[kRT][2], plo[SPLIT ? kRT : 1][2];
 #pragma unroll
     for (int rt = 0; rt < kRT; ++rt) {
-      const float nb = m_run[rt] == -INFINITY ? 0.f : -m_run[rt] * p.scale_log2;
+      const float mb = m_run[rt] == -INFINITY ? 0.f : m_run[rt];
+      float ps = 0.f;
 #pragma unroll
       for (int kh2 = 0; kh2 < 2; ++kh2) {
         float pv[8];
 #pragma unroll
         for (int q = 0; q < 8; ++q)
-          pv[q] = sd::fast_exp2(__builtin_fmaf(sc[rt][2 * kh2 + q / 4][q % 4], p.scale_log2, nb));
+          pv[q] = sd::fast_exp2(sc[rt][2 * kh2 + q / 4][q % 4] - mb);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) ps += pv[q];
         if constexpr (SPLIT) {
           uint32_t hi[4], lo[4];
 #pragma unroll
@@ -351,9 +351,8 @@ void prefill_kernel(PrefillParams p) {
           phi[rt][kh2] = u32x4{sd::pack2<T>(pv[0], pv[1]), sd::pack2<T>(pv[2], pv[3]),
                                sd::pack2<T>(pv[4], pv[5]), sd::pack2<T>(pv[6], pv[7])};
         }
-        lsum[rt] = sd::Elem<T>::mfma(ones, phi[rt][kh2], lsum[rt]);
-        if constexpr (SPLIT) lsum[rt] = sd::Elem<T>::mfma(ones, plo[rt][kh2], lsum[rt]);
       }
+      l_run[rt] += ps;
     }
     // ---- O^T += V^T . P^T; in 32-key half kh2, k-slot 8 lg + j <-> key
     //      32 kh2 + 4 lg + j (j < 4) and 32 kh2 + 16 + 4 lg + j - 4 (j >= 4)
@@ -387,7 +386,7 @@ void prefill_kernel(PrefillParams p) {
   // ---- normalised rows: lane holds O[row lr][dims 16 dt + 4 lg .. +4]
 #pragma unroll
   for (int rt = 0; rt < kRT; ++rt) {
-    const float l = lsum[rt][0];
+    const float l = sd::sum_over_groups(l_run[rt]);
     if (!valid[rt]) continue;
     const float inv = l > 0.f ? 1.f / l : 0.f;
     uint16_t* op = p.out + (q0 + qi[rt]) * p.o_stok +
@@ -487,9 +486,7 @@ extern "C" int sd_prefill_attention(
   p.G = G;
   p.Hkv = num_kv_heads;
   p.total_q = total_q;
-  const float mag = fabsf(scale) * 1.4426950408889634f;
-  p.scale_log2 = mag == 0.f ? 1e-37f : mag;  // (0 would turn a masked score's -inf into NaN)
-  p.q_flip = scale < 0.f ? 0x80008000u : 0u;
+  p.scale_log2 = scale * 1.4426950408889634f;
   p.out = static_cast<uint16_t*>(out);
   p.o_stok = out_stride_tok;
   p.o_shead = out_stride_head;

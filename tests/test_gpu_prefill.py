@@ -156,8 +156,7 @@ def test_attention_layer_prefill_stores_and_attends():
 
 @pytest.mark.parametrize("scale", [-0.08, 0.0, 0.3])
 def test_scale_signs(scale):
-    # the scale enters the exponent's multiply-add, its sign the bits of q; 0.3 makes rows
-    # that a single key dominates
+    # 0.3 makes rows that a single key dominates
     lens = [130, 65]
     q, k, v, cu_q, cu_k = make(lens, lens, 16, 8, seed=21)
     o = ops.prefill_attention(q.to(DEV), k.to(DEV), v.to(DEV), cu_q.to(DEV), cu_k.to(DEV),
@@ -190,3 +189,25 @@ def test_row_strides_past_the_short_offsets():
     vd.copy_(v)
     o = ops.prefill_attention(q.to(DEV), kd, vd, cu_q.to(DEV), cu_k.to(DEV), n, 128 ** -0.5)
     assert_close_attn(to_np(o.float()), ref_varlen(q, k, v, cu_q, cu_k, 128 ** -0.5), what="strides")
+
+
+@pytest.mark.parametrize("dtype,tail,n,rel", [
+    # a weight that fp16 rounds to 0: 2^17 of them are 0.4% of the row's sum
+    (torch.float16, 2.0 ** -25.1, 1 << 17, 2.0 ** -11),
+    # a weight that bf16 rounds down by 0.4%, most of the row's sum; the output is next to 255 / 2048
+    (torch.bfloat16, 2.0 ** -8 * (1 + 0.98 * 2.0 ** -8), 1793, 2.0 ** -9)])
+def test_row_sum_takes_the_weights_before_rounding(dtype, tail, n, rel):
+    # the first key of weight 1 and value 1, n keys of weight `tail` and value 0: the output is
+    # 1 / (1 + n tail), within the half ulp of its own rounding (rel) and 1e-4 for the
+    # exponentials and the fp32 sum; n <= 2^17 additions of one sign, at most 2^-24 each
+    q = torch.zeros((1, 1, 128), dtype=dtype)
+    k = torch.zeros((n + 1, 1, 128), dtype=dtype)
+    v = torch.zeros_like(k)
+    q[..., 0] = 1
+    k[0, :, 0] = 1
+    v[0] = 1
+    cu_q, cu_k = torch.tensor([0, 1], dtype=torch.int32), torch.tensor([0, n + 1], dtype=torch.int32)
+    o = ops.prefill_attention(q.to(DEV), k.to(DEV), v.to(DEV), cu_q.to(DEV), cu_k.to(DEV), 1,
+                              -math.log(tail))
+    err = float((o.double() * (1 + n * tail) - 1).abs().max())
+    assert err <= rel + 1e-4, err
