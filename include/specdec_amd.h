@@ -283,6 +283,15 @@ int sd_paged_attention_store(const void* key, int64_t key_stride_tok, int64_t ke
 size_t sd_w8a16_workspace_size(int64_t M, int64_t N, int64_t K, int32_t group_size);
 
 /*
+ * The route of sd_w8a16_linear for this shape on the current device (host only):
+ * 0 where the row-streaming or 16-row kernels run it (the kernels that the SiLU
+ * and RMSNorm forms below share), else
+ *   K slices | tile weight rows << 8 | tile activation rows << 20
+ * of the tiled kernel. Also 0 for sizes that sd_w8a16_linear refuses.
+ */
+int64_t sd_w8a16_plan(int64_t M, int64_t N, int64_t K, int32_t group_size);
+
+/*
  * W8A16 weight-only linear: y = x @ (w * scale)^T (+ bias).
  * Replaces `int8_linear` with `_int8_dequant_gemm_kernel` and
  * `_splitk_reduce_kernel` (nanovllm/layers/quant.py:165-310).
@@ -298,9 +307,9 @@ size_t sd_w8a16_workspace_size(int64_t M, int64_t N, int64_t K, int32_t group_si
  * whole weight rows through fp32 FMAs, and so does one row on larger weights
  * (the lm_head), with batches of 4 rows dealt to the waves in turn; other
  * shapes run the 16-row MFMA kernel (the SiLU and RMSNorm forms below follow the
- * same rule), and past 16 rows most run a tiled MFMA kernel (small layers at
- * up to 128 rows, and more than 32 Mi weights of K <= 1024 at up to 32 rows, stay on
- * the former). Supported: K % 64 == 0,
+ * same rule), and past 16 rows most run a tiled MFMA kernel (small layers and
+ * vocabulary heads at a few rows stay on the former: sd_w8a16_plan).
+ * Supported: K % 64 == 0,
  * group_size 0 or a multiple of 64 dividing K; N < 2^24 rows, a row stride
  * below 2^24 bytes and N * w_stride_n < 2^32 bytes (the MFMA kernel forms a
  * row's byte offset with one 24 x 24-bit multiply-add; SD_ERR_UNSUPPORTED

@@ -64,6 +64,8 @@ struct W8GemmArgs {
 // the 16-row kernels. A function of the sizes alone, so every form of the call
 // (plain, SiLU, RMSNorm) sums in the same order.
 int w8a16_gemm_splits(int64_t M, int64_t N, int64_t K, int32_t group);
+// The tile and slices as sd_w8a16_plan returns them.
+int64_t w8a16_gemm_plan_code(int64_t M, int64_t N, int64_t K, int32_t group);
 // Bytes of fp32 partial sums (0 with one slice).
 size_t w8a16_gemm_workspace(int64_t M, int64_t N, int64_t K, int32_t group);
 // Whether the kernel can run this call (its sizes, LDS scale table and 32-bit row offsets),

@@ -1556,11 +1556,20 @@ int launch_rows_any(const W8Params& p, int mode, hipStream_t st) {
 
 }  // namespace
 
+namespace {
+// Sizes that sd_w8a16_linear runs; others have no plan.
+bool w8_sizes_ok(int64_t M, int64_t N, int64_t K, int32_t group_size) {
+  return M > 0 && N > 0 && K > 0 && K % 64 == 0 && group_size >= 0 && group_size % 64 == 0 &&
+         M <= (1ll << 30) && N <= (1ll << 30) && K <= (1ll << 30) && !(group_size && K % group_size);
+}
+}  // namespace
+
 extern "C" size_t sd_w8a16_workspace_size(int64_t M, int64_t N, int64_t K, int32_t group_size) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % 64 || group_size < 0 || group_size % 64 || M > (1ll << 30) ||
-      N > (1ll << 30) || K > (1ll << 30) || (group_size && K % group_size))
-    return 0;  // nothing to run, or refused by sd_w8a16_linear
-  return sd::w8a16_gemm_workspace(M, N, K, group_size);
+  return w8_sizes_ok(M, N, K, group_size) ? sd::w8a16_gemm_workspace(M, N, K, group_size) : 0;
+}
+
+extern "C" int64_t sd_w8a16_plan(int64_t M, int64_t N, int64_t K, int32_t group_size) {
+  return w8_sizes_ok(M, N, K, group_size) ? sd::w8a16_gemm_plan_code(M, N, K, group_size) : 0;
 }
 
 namespace {

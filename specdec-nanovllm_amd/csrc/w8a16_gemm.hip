@@ -513,19 +513,53 @@ GemmParams params(const sd::W8GemmArgs& a, int splits, void* workspace) {
 
 namespace sd {
 
-// From 17 rows up, except where the 16-row kernels measured faster: layers of at most
-// 8 Mi weights while M N K <= 5.4e8 and M <= 128 (one launch, K split inside a workgroup:
-// 1024 x 2048 at M = 56 6.1 us there against 9.2 here, at M = 128 10.0 against 10.5, at
-// M = 256 16.8 against 12.3; 6144 x 1024 at M = 56 9.2 against 11.0, at M = 128 13.6
-// against 12.0). Per group the same line; 2560 x 9728 at M = 17 is 20 us there, 14 here.
-// And except the vocabulary head at up to 32 rows (K <= 1024, more than 32 Mi weights), which
-// the 16-row kernel reads as whole rows, once per block of up to 32 staged rows: 39.4 us there,
-// 43.9 here (norm included, 151936 x 1024); at M = 56 55.4 there, 49.4 here.
+// From 17 rows up, except where the 16-row kernels are faster. Both were timed from graphs
+// at 6481 shapes (M 17 - 1024, N 64 - 262144, K 64 - 9728, per channel and in groups of 128),
+// weights rotating through HBM; "there" is the 16-row kernel:
+//  * layers of at most 8 Mi weights while M <= 128 and M N K <= 5.4e8 (one launch, K split
+//    inside a workgroup): 1024 x 2048 at M = 56 6.1 us there against 9.2 here, at M = 128
+//    10.0 against 10.5; 6144 x 1024 at M = 56 9.2 against 11.0, at M = 128 13.6 against 12.0;
+//  * few 16 x 16 output tiles, whatever M: the tiles here are too few for the device, and a
+//    second launch for K slices costs more than it saves. Up to three tiles per CU at K <= 1024
+//    (256 x 1024 at M = 512 5.1 us there, 6.6 here; 1024 x 1024 at M = 192 6.2 and 7.1, at
+//    M = 256, four per CU, 6.9 and 7.0), one per CU up to K = 3072 (256 x 2048 at M = 256 5.7
+//    and 7.2; past 512 rows a 16-row grid of that few columns is too narrow: 64 x 2048 at
+//    M = 768 18.4 and 6.9). Per group six and four below K = 512, one up to K = 2048
+//    (1024 x 1024 at M = 256 8.4 and 10.0; 6144 x 1024 at M = 64 10.1 and 13.2). From K = 256:
+//    a few steps do not split there (256 x 128 at M = 256 6.1 and 4.0);
+//  * many rows of few columns (vocabulary heads), read there as whole rows against the staged
+//    activations, here in tiles of few steps: up to 32 rows from 64 Ki weight rows at
+//    K <= 1024 (151936 x 1024 at M = 17 37.5 and 39.5, 65536 x 1024 17.7 and 20.7, but
+//    40000 x 1024 16.4 and 14.9), up to 64 from 96 Ki rows while M K <= 36 Ki and within
+//    100 Mi weights (100000 x 256 at M = 48 14.9 and 20.1, x 768 28.7 and 32.6; 262144 x 512
+//    at M = 48, past that, 41.8 and 40.2). Per group up to 32 rows at K <= 512 from 32 Mi weights
+//    (65536 x 512 at M = 24 12.1 and 14.4).
+// What is left: 129 - 224 rows of K <= 256 at 12288 columns and more are 5 - 13% slower here,
+// where 64-row blocks fit the row count better than these tiles.
+bool stays_on_16_rows(int64_t M, int64_t N, int64_t K, int32_t group) {
+  constexpr int64_t kKi = 1024, kMi = 1024 * 1024;
+  if (M <= 16) return true;
+  if (M <= 128 && N * K <= 8 * kMi && static_cast<double>(M) * N * K <= 5.4e8) return true;
+  const int64_t cus = device_cus(), tiles = (M + 15) / 16 * ((N + 15) / 16);
+  if (K >= 256 && K <= 1024) {
+    if (tiles <= (group == 0 ? 3 : K < 512 ? 4 : 6) * cus) return true;
+  } else if (K > 1024 && K <= (group ? 2048 : 3072)) {
+    if (M <= 512 && tiles <= cus) return true;
+  }
+  if (group) return M <= 32 && K <= 512 && N * K >= 32 * kMi;
+  return (M <= 32 && K <= 1024 && N >= 64 * kKi) ||
+         (M <= 64 && M * K <= 36 * kKi && N >= 96 * kKi && N * K <= 100 * kMi);
+}
+
 int w8a16_gemm_splits(int64_t M, int64_t N, int64_t K, int32_t group) {
-  if (M <= 16) return 0;
-  if (M <= 32 && K <= 1024 && group == 0 && N * K > (int64_t{32} << 20)) return 0;
-  if (M <= 128 && N * K <= (int64_t{8} << 20) && static_cast<double>(M) * N * K <= 5.4e8) return 0;
-  return plan_for(M, N, K, group).splits;
+  return stays_on_16_rows(M, N, K, group) ? 0 : plan_for(M, N, K, group).splits;
+}
+
+int64_t w8a16_gemm_plan_code(int64_t M, int64_t N, int64_t K, int32_t group) {
+  if (stays_on_16_rows(M, N, K, group)) return 0;
+  const Plan pl = plan_for(M, N, K, group);
+  return pl.splits | static_cast<int64_t>(kShapes[pl.tile].bn) << 8 |
+         static_cast<int64_t>(kShapes[pl.tile].bm) << 20;
 }
 
 size_t w8a16_gemm_workspace(int64_t M, int64_t N, int64_t K, int32_t group) {

@@ -332,6 +332,15 @@ def w8a16_linear(x: torch.Tensor, qweight: torch.Tensor, scale: torch.Tensor,
 
 
 
+def _many_rows(M: int, N: int, K: int, group_size: int, dev: torch.device) -> bool:
+    """Whether the plain linear leaves the 16-row kernels that the fused forms share
+    (never up to 16 rows; past them a matter of sizes and compute units)."""
+    if M <= 16 or dev.type != "cuda":
+        return False
+    with _lib.on_device(dev):
+        return _lib.load().sd_w8a16_plan(M, N, K, int(group_size)) != 0
+
+
 def w8a16_silu_linear(gate_up: torch.Tensor, qweight: torch.Tensor, scale: torch.Tensor,
                       bias: torch.Tensor | None = None, group_size: int = 0,
                       out: torch.Tensor | None = None) -> torch.Tensor:
@@ -339,9 +348,9 @@ def w8a16_silu_linear(gate_up: torch.Tensor, qweight: torch.Tensor, scale: torch
     (layers/activation.py:6-11 then the W8A16 linear). gate_up: (..., 2K); the
     activation is SiluAndMul's, bit for bit. One launch while the fused form
     stages its activation rows in LDS (min(M, 16) (2K + 16) <= 33,024 bytes)
-    and the plain linear stays on the 16-row kernels it shares (up to 16 rows,
-    or 128 on at most 8 Mi weights), the two separate launches otherwise (the
-    faster of the two there)."""
+    and the plain linear stays on the 16-row kernels it shares (sd_w8a16_plan),
+    up to 128 rows (every workgroup repeats the SiLU of its rows: 1024 x 1024 at
+    192 rows 17.4 us, 9.3 in two launches); the two separate launches otherwise."""
     assert qweight.dtype == torch.int8 and qweight.dim() == 2
     N, K = qweight.shape
     g2 = gate_up.reshape(-1, gate_up.shape[-1])
@@ -355,7 +364,8 @@ def w8a16_silu_linear(gate_up: torch.Tensor, qweight: torch.Tensor, scale: torch
         assert sc.numel() == N * (K // group_size), "per-group scale must be (N, K // group_size)"
     else:
         assert sc.numel() == N, "per-channel scale must have N entries"
-    if min(M, 16) * (2 * K + 16) > 33024 or M > (16 if N * K > 8 << 20 else 128):
+    if min(M, 16) * (2 * K + 16) > 33024 or M > 128 or \
+            _many_rows(M, N, K, group_size, g2.device):
         y = w8a16_linear(silu_mul(g2), qw, sc, bias, group_size, out)
         return y.view(*gate_up.shape[:-1], N)
     b = None if bias is None else bias.to(gate_up.dtype).contiguous()

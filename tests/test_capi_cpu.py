@@ -105,9 +105,31 @@ def test_workspace_queries():
     assert nv == (ev * 8 + 255) // 256 * 256 + ev * 128 * 4
     assert lib.sd_paged_attention_workspace_size(32, 1, 32, 8, 128, 4096, 0) > 0
     assert lib.sd_paged_attention_workspace_size(0, 1, 32, 8, 128, 4096, 0) == 0
-    # W8A16 is one launch for every shape (K splits are added inside a workgroup)
+    # W8A16 up to 16 rows and in small layers: K splits are added inside a workgroup
     for M, N, K in [(1, 151936, 1024), (1, 1024, 3072), (56, 4096, 1024)]:
         assert lib.sd_w8a16_workspace_size(M, N, K, 0) == 0
+
+
+@pytest.mark.parametrize("M,N,K,group", [
+    (16, 19456, 2560, 0), (56, 1024, 2048, 0), (128, 6144, 512, 0),  # up to 16 rows, small layers
+    (192, 1024, 1024, 0), (512, 256, 1024, 0), (256, 256, 2048, 0), (256, 256, 3072, 0),
+    (256, 1024, 1024, 128), (64, 6144, 1024, 128), (32, 12288, 1024, 128), (512, 64, 2048, 128),
+    (17, 151936, 64, 0), (32, 65536, 512, 0), (32, 151936, 1024, 0), (64, 100000, 512, 0),
+    (48, 100000, 768, 0), (24, 65536, 512, 128), (32, 262144, 128, 128)])
+def test_w8a16_routes_to_the_16_row_kernels(M, N, K, group):
+    # sizes that measured faster on them than in tiles
+    assert _lib.load().sd_w8a16_plan(M, N, K, group) == 0
+    assert _lib.load().sd_w8a16_workspace_size(M, N, K, group) == 0
+
+
+@pytest.mark.parametrize("M,N,K,group", [
+    (17, 19456, 2560, 0), (56, 2560, 9728, 0), (256, 1024, 2048, 0), (768, 64, 2048, 0),
+    (256, 256, 128, 0), (17, 40000, 1024, 0), (33, 151936, 1024, 0), (64, 49152, 512, 0),
+    (384, 6144, 512, 128), (17, 151936, 1024, 128)])
+def test_w8a16_routes_to_tiles(M, N, K, group):
+    plan = _lib.load().sd_w8a16_plan(M, N, K, group)
+    assert plan & 0xff in (1, 2, 3, 4, 6, 8, 12, 16)  # K slices
+    assert (plan >> 8) & 0xfff in (64, 80, 96, 128, 256) and plan >> 20 in (32, 64, 128, 256)
 
 
 def test_ops_refuse_cpu_tensors():

@@ -162,6 +162,8 @@ def test_errors():
                                           (2, 1024, 1024, 0, torch.bfloat16),
                                           (7, 1024, 3072, 0, torch.float16),
                                           (56, 1024, 3072, 0, torch.bfloat16),
+                                          (192, 1024, 1024, 0, torch.bfloat16),
+                                          (300, 520, 1024, 128, torch.float16),
                                           (3, 33000, 1024, 0, torch.bfloat16),
                                           (20, 33000, 1024, 128, torch.float16),
                                           (40, 33000, 1024, 0, torch.bfloat16),
