@@ -59,11 +59,12 @@ struct W8GemmArgs {
   int32_t dtype;
 };
 
-// K slices of the many-row kernel for this shape (1, 2, 4, 8 or 16; slice s covers
-// the 64-column steps [s K/64 / n, (s + 1) K/64 / n)), or 0: the shape stays on
-// the 16-row kernels. A function of the sizes alone, so every form of the call
-// (plain, SiLU, RMSNorm) sums in the same order.
-int w8a16_gemm_splits(int64_t M, int64_t N, int64_t K, int32_t group);
+// K slices of the many-row kernel for this shape (1, 2, 3, 4, 6, 8, 12 or 16), or 0: the
+// shape stays on the 16-row kernels. Slice s of n covers the stages [s S / n, (s + 1) S / n)
+// of S = K / 64 / *kb stages of *kb 64-column steps (1 or 2). A function of the sizes and the
+// device's compute units, so that the forms that stay on the 16-row kernels (SiLU, RMSNorm)
+// can add the same slices in the same order.
+int w8a16_gemm_splits(int64_t M, int64_t N, int64_t K, int32_t group, int* kb);
 // The tile and slices as sd_w8a16_plan returns them.
 int64_t w8a16_gemm_plan_code(int64_t M, int64_t N, int64_t K, int32_t group);
 // Bytes of fp32 partial sums (0 with one slice).

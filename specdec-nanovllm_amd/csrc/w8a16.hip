@@ -49,6 +49,7 @@ struct W8Params {
   int64_t ys;
   int32_t M, N, K;
   int32_t nks;     // K / 64
+  int32_t kb, nst; // K slices start on whole stages of kb steps; nst = nks / kb
   int32_t groups;  // row groups of 16 NT rows
   int32_t xpitch;  // bytes per activation row in LDS (staged activations only)
   int32_t xbytes;  // XL: bytes of staged activation rows; the scale table follows
@@ -140,9 +141,9 @@ __global__ __launch_bounds__(NWV * 64) void w8a16_kernel(W8Params p) {
 
   // K steps of this wave: [ks, ke); every wave of a row group runs the same
   // number of chunks (so the LDS reduction lines up), short ones skip steps.
-  const int ks = static_cast<int>(static_cast<int64_t>(kw) * p.nks / KW);
-  const int ke = static_cast<int>(static_cast<int64_t>(kw + 1) * p.nks / KW);
-  const int nchunks = ((p.nks + KW - 1) / KW + U - 1) / U;
+  const int ks = p.kb * static_cast<int>(static_cast<int64_t>(kw) * p.nst / KW);
+  const int ke = p.kb * static_cast<int>(static_cast<int64_t>(kw + 1) * p.nst / KW);
+  const int nchunks = (p.kb * ((p.nst + KW - 1) / KW) + U - 1) / U;
 
   // row groups of this wave: g0, g0 + gstride, ... (ngroups of them). Grid-stride
   // over the whole matrix, or (CONTIG) a contiguous range per workgroup whose
@@ -1226,11 +1227,12 @@ struct RowsPlan {
 struct W8Plan {
   int MT, NT, KW, mblocks, groups, grid;
   int gemm;  // K slices of the many-row kernel (plain calls run it), 0: it stays out
+  int kb;    // 64-column steps per stage: slices start on whole ones
 };
 
 W8Plan make_plan(int64_t M, int64_t N, int64_t K, int32_t group) {
   W8Plan pl;
-  pl.gemm = sd::w8a16_gemm_splits(M, N, K, group);
+  pl.gemm = sd::w8a16_gemm_splits(M, N, K, group, &pl.kb);
   // Activation rows in blocks of 16 (MT = 1), 32 (MT = 2) or 64 (MT = 4) along
   // grid.y. Every block streams the whole weight matrix, and a second block
   // only hits L2 while it runs in step with the first: with the weight loads
@@ -1249,7 +1251,7 @@ W8Plan make_plan(int64_t M, int64_t N, int64_t K, int32_t group) {
   // chunks each (a narrow layer has too few tiles to fill the GPU with 4:
   // N = 1024 is 64 workgroups), else 4.
   // Where plain calls run the many-row kernel, the SiLU and RMSNorm forms keep to its
-  // K slices (the same sums).
+  // K slices, one wave each (the same sums).
   if (pl.gemm == 1 || (pl.gemm == 0 && (nr * pl.mblocks >= 8ll * cus || nks < 4))) {
     pl.KW = 1;
     // 16-row groups balance better over the waves (lm_head M = 1: 29.0 vs
@@ -1414,6 +1416,11 @@ int launch_kw(const W8Params& p, const W8Plan& pl, dim3 grid, hipStream_t st) {
   }
 }
 
+int no_slices(int n) {  // a plan that no kernel instance was built for
+  sd::set_error("w8a16: no kernel for %d K slices", n);
+  return SD_ERR_UNSUPPORTED;
+}
+
 template <typename T, int MODE, bool FLOOR = false>
 int launch_all(const W8Params& p, const W8Plan& pl, hipStream_t st) {
   int rc;
@@ -1422,9 +1429,13 @@ int launch_all(const W8Params& p, const W8Plan& pl, hipStream_t st) {
     switch (pl.KW) {
       case 1: rc = launch_kw<T, false, 1, MODE, FLOOR>(p, pl, grid, st); break;
       case 2: rc = launch_kw<T, false, 2, MODE, FLOOR>(p, pl, grid, st); break;
-      case 16: rc = launch_kw<T, false, 16, MODE, FLOOR>(p, pl, grid, st); break;
+      case 3: rc = launch_kw<T, false, 3, MODE, FLOOR>(p, pl, grid, st); break;
+      case 4: rc = launch_kw<T, false, 4, MODE, FLOOR>(p, pl, grid, st); break;
+      case 6: rc = launch_kw<T, false, 6, MODE, FLOOR>(p, pl, grid, st); break;
       case 8: rc = launch_kw<T, false, 8, MODE, FLOOR>(p, pl, grid, st); break;
-      default: rc = launch_kw<T, false, 4, MODE, FLOOR>(p, pl, grid, st); break;
+      case 12: rc = launch_kw<T, false, 12, MODE, FLOOR>(p, pl, grid, st); break;
+      case 16: rc = launch_kw<T, false, 16, MODE, FLOOR>(p, pl, grid, st); break;
+      default: rc = no_slices(pl.KW); break;
     }
   } else {
     if constexpr (FLOOR) {
@@ -1434,9 +1445,13 @@ int launch_all(const W8Params& p, const W8Plan& pl, hipStream_t st) {
       switch (pl.KW) {
         case 1: rc = launch_kw<T, true, 1, MODE>(p, pl, grid, st); break;
         case 2: rc = launch_kw<T, true, 2, MODE>(p, pl, grid, st); break;
-        case 16: rc = launch_kw<T, true, 16, MODE>(p, pl, grid, st); break;
+        case 3: rc = launch_kw<T, true, 3, MODE>(p, pl, grid, st); break;
+        case 4: rc = launch_kw<T, true, 4, MODE>(p, pl, grid, st); break;
+        case 6: rc = launch_kw<T, true, 6, MODE>(p, pl, grid, st); break;
         case 8: rc = launch_kw<T, true, 8, MODE>(p, pl, grid, st); break;
-        default: rc = launch_kw<T, true, 4, MODE>(p, pl, grid, st); break;
+        case 12: rc = launch_kw<T, true, 12, MODE>(p, pl, grid, st); break;
+        case 16: rc = launch_kw<T, true, 16, MODE>(p, pl, grid, st); break;
+        default: rc = no_slices(pl.KW); break;
       }
     }
   }
@@ -1675,6 +1690,8 @@ int run_w8a16(const void* x, int64_t x_stride_m, int64_t up, const NormArgs& nor
   p.N = static_cast<int32_t>(N);
   p.K = static_cast<int32_t>(K);
   p.nks = static_cast<int32_t>(K / 64);
+  p.kb = pl.kb;
+  p.nst = p.nks / pl.kb;
   p.groups = pl.groups;
   // staged activation rows (wide path): K * 2 bytes + a 16-byte pad per row, so
   // that the 16 rows of a B-operand read start 4 banks apart

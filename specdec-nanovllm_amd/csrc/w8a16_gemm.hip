@@ -24,9 +24,10 @@
 //
 // Sums: one fp32 accumulator per output over the K slice, in ascending k and with the
 // operand order of w8a16_kernel (lane group g holds k = 16 g .. 16 g + 15 of a step, two
-// MFMAs), so a shape gives the same bits on either kernel with the same K slices. With
-// several slices each writes its fp32 partials and w8a16_gemm_reduce adds them in slice
-// order, then scales and rounds (partial sums stay 32-bit).
+// MFMAs), so a shape gives the same bits on either kernel with the same K slices (which
+// start on whole stages). With several slices each writes its fp32 partials and
+// w8a16_gemm_reduce adds them in slice order, then scales and rounds (partial sums stay
+// 32-bit).
 #include "w8a16.h"
 
 namespace {
@@ -551,8 +552,12 @@ bool stays_on_16_rows(int64_t M, int64_t N, int64_t K, int32_t group) {
          (M <= 64 && M * K <= 36 * kKi && N >= 96 * kKi && N * K <= 100 * kMi);
 }
 
-int w8a16_gemm_splits(int64_t M, int64_t N, int64_t K, int32_t group) {
-  return stays_on_16_rows(M, N, K, group) ? 0 : plan_for(M, N, K, group).splits;
+int w8a16_gemm_splits(int64_t M, int64_t N, int64_t K, int32_t group, int* kb) {
+  *kb = 1;
+  if (stays_on_16_rows(M, N, K, group)) return 0;
+  const Plan pl = plan_for(M, N, K, group);
+  *kb = kShapes[pl.tile].kb;
+  return pl.splits;
 }
 
 int64_t w8a16_gemm_plan_code(int64_t M, int64_t N, int64_t K, int32_t group) {
@@ -563,13 +568,15 @@ int64_t w8a16_gemm_plan_code(int64_t M, int64_t N, int64_t K, int32_t group) {
 }
 
 size_t w8a16_gemm_workspace(int64_t M, int64_t N, int64_t K, int32_t group) {
-  const int splits = w8a16_gemm_splits(M, N, K, group);
+  int kb;
+  const int splits = w8a16_gemm_splits(M, N, K, group, &kb);
   if (splits <= 1) return 0;
   return static_cast<size_t>(splits) * static_cast<size_t>(M) * static_cast<size_t>(pitch_of(N)) * sizeof(float);
 }
 
 bool w8a16_gemm_fits(const W8GemmArgs& a, const void* workspace, size_t workspace_bytes, int* splits) {
-  *splits = w8a16_gemm_splits(a.M, a.N, a.K, a.group);
+  int kb;
+  *splits = w8a16_gemm_splits(a.M, a.N, a.K, a.group, &kb);
   if (*splits == 0) return false;
   // without the partial sums' workspace: one slice
   if (*splits > 1 && (!workspace || !aligned16(workspace) ||

@@ -164,6 +164,14 @@ def test_errors():
                                           (56, 1024, 3072, 0, torch.bfloat16),
                                           (192, 1024, 1024, 0, torch.bfloat16),
                                           (300, 520, 1024, 128, torch.float16),
+                                          # past the 16-row kernels' sizes: the tiled kernel's
+                                          # K slices (3, 6, 12, 8, two-step stages; per group)
+                                          (256, 1024, 3072, 0, torch.bfloat16),
+                                          (56, 2560, 9728, 0, torch.float16),
+                                          (18, 2570, 9728, 0, torch.bfloat16),
+                                          (33, 2560, 4096, 0, torch.float16),
+                                          (200, 1030, 2048, 128, torch.bfloat16),
+                                          (640, 4096, 576, 0, torch.bfloat16),
                                           (3, 33000, 1024, 0, torch.bfloat16),
                                           (20, 33000, 1024, 128, torch.float16),
                                           (40, 33000, 1024, 0, torch.bfloat16),
@@ -208,7 +216,9 @@ def test_silu_linear_is_silu_mul_then_linear(M, N, K, gs, act):
                                               (13, 2048, 576, 0, torch.bfloat16, True),
                                               (5, 4096, 1024, 0, torch.float16, False),
                                               (16, 512, 64, 0, torch.bfloat16, True),
-                                              (11, 6144, 1024, 0, torch.bfloat16, True)])
+                                              (11, 6144, 1024, 0, torch.bfloat16, True),
+                                              # the tiled kernel's K slices
+                                              (17, 9216, 960, 0, torch.bfloat16, True)])
 def test_rmsnorm_linear_is_rmsnorm_then_linear(M, N, K, gs, act, res):
     # add + RMSNorm formed while staging: bit-identical to rmsnorm then the
     # linear, residual_out identical to rmsnorm's (one row block per 16 or 32
