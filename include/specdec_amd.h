@@ -406,7 +406,9 @@ int sd_w8a16_rmsnorm_linear(const void* x, int64_t x_stride_m, const void* resid
  * 32 MiB of weights, N even) a wave streams gate row i together with up row
  * I + i; on the K-split path of sd_w8a16_linear (narrow layers, per-channel
  * scale, N a multiple of 32) a workgroup takes gate tile g and up tile g with
- * the plain projection's K split, so the sums are the projection's own. The
+ * the plain projection's K split, so the sums are the projection's own (past 16
+ * rows those of the tiled kernel; the two calls are faster where it runs:
+ * sd_w8a16_plan not 0). The
  * down projection then reads the activated rows with no SiLU of its own.
  * Other shapes return SD_ERR_UNSUPPORTED (the caller runs the two calls).
  * y: (M, N / 2) dtype, sharing no byte with x, residual or residual_out.

@@ -112,7 +112,8 @@ using sd::load_scale;
 // every loaded weight word folded into a register instead of the staging through
 // the LDS tile, the MFMAs and the epilogue; no output.
 template <typename T, int MT, int NT, int KW, int U, bool PER_GROUP, bool CONTIG = false,
-          int D = 2, bool XL = false, int MODE = 0, int NWV = kWaves, bool FLOOR = false>
+          int D = 2, bool XL = false, int MODE = 0, int NWV = kWaves, bool FLOOR = false,
+          bool PAIRED = false>
 __global__ __launch_bounds__(NWV * 64) void w8a16_kernel(W8Params p) {
   constexpr bool SL = MODE == 1;
   constexpr bool NM = MODE == 2;
@@ -172,10 +173,11 @@ __global__ __launch_bounds__(NWV * 64) void w8a16_kernel(W8Params p) {
   auto srow = [&](int g, int r) {  // scale-table row of row r of group g (this wave's)
     return (sub * p.ngmax + (g - g0) / gstride) * RG + r;
   };
-  // pr: gate_up with the SiLU epilogue on the K-split path. Group g is gate tile
+  // pr: gate_up with the SiLU epilogue on the K-split path (PAIRED: by whole-row waves,
+  // where the tiled kernel's plan has one slice). Group g is gate tile
   // g (weight rows 16 g ..) and up tile g (rows pair + 16 g ..); its 16 outputs
   // are bf16(bf16(silu(gate)) * up) of the rows the projection would write.
-  constexpr bool PRC = KW > 1 && NT == 2 && MODE != 1 && !PER_GROUP;
+  constexpr bool PRC = (KW > 1 || PAIRED) && NT == 2 && MODE != 1 && !PER_GROUP;
   const bool pr = PRC && p.pair > 0;
   const int nrows = pr ? 2 * p.pair : p.N;  // weight rows
   auto wrow = [&](int g, int r) {  // weight row of row r (0 .. RG - 1) of group g
@@ -1228,6 +1230,7 @@ struct W8Plan {
   int MT, NT, KW, mblocks, groups, grid;
   int gemm;  // K slices of the many-row kernel (plain calls run it), 0: it stays out
   int kb;    // 64-column steps per stage: slices start on whole ones
+  bool narrow;  // too few rows for whole-row waves: gate_up has its SiLU epilogue
 };
 
 W8Plan make_plan(int64_t M, int64_t N, int64_t K, int32_t group) {
@@ -1252,7 +1255,8 @@ W8Plan make_plan(int64_t M, int64_t N, int64_t K, int32_t group) {
   // N = 1024 is 64 workgroups), else 4.
   // Where plain calls run the many-row kernel, the SiLU and RMSNorm forms keep to its
   // K slices, one wave each (the same sums).
-  if (pl.gemm == 1 || (pl.gemm == 0 && (nr * pl.mblocks >= 8ll * cus || nks < 4))) {
+  pl.narrow = nr * pl.mblocks < 8ll * cus && nks >= 4;
+  if (pl.gemm == 1 || (pl.gemm == 0 && !pl.narrow)) {
     pl.KW = 1;
     // 16-row groups balance better over the waves (lm_head M = 1: 29.0 vs
     // 30.0 us); from M = 8 up, 32-row groups reuse each activation read twice
@@ -1336,7 +1340,8 @@ constexpr size_t w8_static_lds() {
          static_cast<size_t>(KW > 1 ? KW - 1 : 1) * (NT * MT * 4) * 64 * 4;
 }
 
-template <typename T, int MT, int NT, int KW, bool PG, int MODE, bool FLOOR = false>
+template <typename T, int MT, int NT, int KW, bool PG, int MODE, bool FLOOR = false,
+          bool PAIRED = false>
 int launch_k(const W8Params& p, dim3 grid, hipStream_t st) {
   // 64-k steps per chunk: 2 where a wave's K slice is a few steps (8 or 16
   // slices) or the chunk covers 32 rows
@@ -1359,7 +1364,7 @@ int launch_k(const W8Params& p, dim3 grid, hipStream_t st) {
       // 8-step chunks through the tile at one workgroup per CU: 77.8 us)
       constexpr int UX = MT >= 2 ? 2 : U;
       constexpr int NSUB = NWV / KW;
-      auto kern = w8a16_kernel<T, MT, NT, KW, UX, PG, false, 2, true, MODE, NWV, FLOOR>;
+      auto kern = w8a16_kernel<T, MT, NT, KW, UX, PG, false, 2, true, MODE, NWV, FLOOR, PAIRED>;
       // occupancy from the activation rows; the scale table adds a few KB (per
       // channel: 16 B per row of the workgroup)
       unsigned cap = static_cast<unsigned>(sd::device_cus() * resident_wgs_xl(kern, xbytes, NTH)) /
@@ -1385,7 +1390,7 @@ int launch_k(const W8Params& p, dim3 grid, hipStream_t st) {
                   "staging LDS", static_cast<int>(p.M < MT * 16 ? p.M : MT * 16), p.K);
     return SD_ERR_UNSUPPORTED;
   } else {
-    auto kern = w8a16_kernel<T, MT, NT, KW, U, PG, false, 2, false, MODE, NWV, FLOOR>;
+    auto kern = w8a16_kernel<T, MT, NT, KW, U, PG, false, 2, false, MODE, NWV, FLOOR, PAIRED>;
     // exactly one resident set of workgroups over all activation blocks (a
     // partial second round would leave most of the GPU idle at the end), grid.x
     // a multiple of 8 so that block (x, y) shares an XCD (and its L2) with (x, 0)
@@ -1400,6 +1405,10 @@ int launch_k(const W8Params& p, dim3 grid, hipStream_t st) {
 template <typename T, bool PG, int KW, int MODE, bool FLOOR = false>
 int launch_kw(const W8Params& p, const W8Plan& pl, dim3 grid, hipStream_t st) {
   if constexpr (KW == 1) {
+    if (p.pair > 0) {
+      if constexpr (!PG && MODE != 1 && !FLOOR) return launch_k<T, 1, 2, 1, PG, MODE, false, true>(p, grid, st);
+      else return SD_ERR_UNSUPPORTED;
+    }
     switch (pl.MT * 8 + pl.NT) {
       case 1 * 8 + 1: return launch_k<T, 1, 1, 1, PG, MODE, FLOOR>(p, grid, st);
       case 1 * 8 + 2: return launch_k<T, 1, 2, 1, PG, MODE, FLOOR>(p, grid, st);
@@ -1711,9 +1720,10 @@ int run_w8a16(const void* x, int64_t x_stride_m, int64_t up, const NormArgs& nor
   if (pair) {
     // the row-streaming path (one or two rows), or the K-split tiled path with
     // the plain projection's plan (same K split, so the same sums), per-channel
-    // scales and whole 16-row tiles of pairs
+    // scales and whole 16-row tiles of pairs. Past 16 rows that is the tiled kernel's
+    // split; with one slice a wave takes the whole K of a pair of tiles.
     const bool rows = N % 2 == 0 && rows_eligible(p, true);
-    const bool tiled = N % 32 == 0 && pl.KW > 1 && pl.gemm == 0 && group_size == 0 && mode != 1;
+    const bool tiled = N % 32 == 0 && pl.narrow && group_size == 0 && mode != 1;
     if (!rows && !tiled) {
       sd::set_error("w8a16_gate_up_silu: the SiLU epilogue runs on the row-streaming path "
                     "(one or two rows, M * ceil(K / 1024) <= 4, per-channel scales, at most "
@@ -1729,9 +1739,11 @@ int run_w8a16(const void* x, int64_t x_stride_m, int64_t up, const NormArgs& nor
       return launch_rows_any<_Float16>(p, mode, st);
     }
     W8Plan pp = pl;
+    pp.MT = 1;
     pp.NT = 2;
+    pp.mblocks = static_cast<int>((M + 15) / 16);
     pp.groups = static_cast<int>(N / 32);
-    pp.grid = pp.groups;
+    pp.grid = pp.KW > 1 ? pp.groups : (pp.groups + kWaves - 1) / kWaves;
     p.groups = pp.groups;
     if (mode == 2) {
       if (dtype == SD_BF16) return launch_all<__bf16, 2>(p, pp, st);

@@ -540,15 +540,17 @@ def w8a16_gate_up_silu(x: torch.Tensor, qweight: torch.Tensor, scale: torch.Tens
                                 K, float(eps), _lib.dtype_code(x.dtype), _lib.stream_ptr(dev))
         _lib.check(rc)
         ra = roa = nwa = None
-    with _lib.on_device(dev):
-        rc = lib.sd_w8a16_gate_up_silu(
-            xa.data_ptr(), xa.stride(0), _ptr(ra), 0 if ra is None else ra.stride(0),
-            _ptr(roa), 0 if roa is None else roa.stride(0), _ptr(nwa), float(eps),
-            qw.data_ptr(), qw.stride(0), sc.data_ptr(), _lib.dtype_code(sc.dtype), _ptr(b),
-            y.data_ptr(), y.stride(0), M, N, K, _lib.dtype_code(x.dtype), _lib.stream_ptr(dev))
+    rc = _lib.SD_ERR_UNSUPPORTED  # past the 16-row kernels: the tiled projection first
+    if not _many_rows(M, N, K, 0, dev):
+        with _lib.on_device(dev):
+            rc = lib.sd_w8a16_gate_up_silu(
+                xa.data_ptr(), xa.stride(0), _ptr(ra), 0 if ra is None else ra.stride(0),
+                _ptr(roa), 0 if roa is None else roa.stride(0), _ptr(nwa), float(eps),
+                qw.data_ptr(), qw.stride(0), sc.data_ptr(), _lib.dtype_code(sc.dtype), _ptr(b),
+                y.data_ptr(), y.stride(0), M, N, K, _lib.dtype_code(x.dtype), _lib.stream_ptr(dev))
     if rc == _lib.SD_ERR_UNSUPPORTED and (nwa is None or (K % 8 == 0 and K <= 8192)):
-        # neither the row-streaming nor the K-split path: the projection, then
-        # the SiLU launch
+        # neither the row-streaming nor the K-split path (or a faster tiled
+        # projection): the projection, then the SiLU launch
         if nwa is None:
             gu = w8a16_linear(xa, qw, sc, b)
         else:

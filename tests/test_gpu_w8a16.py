@@ -358,6 +358,40 @@ def test_gate_up_silu_is_linear_then_silu_mul(M, N, K, act, norm, res):
         assert torch.equal(ro, ro_two)
 
 
+@pytest.mark.parametrize("M,N,K,act,norm", [(88, 6144, 1024, torch.bfloat16, False),  # one slice
+                                            (88, 6144, 1024, torch.float16, True),
+                                            (81, 4128, 2560, torch.bfloat16, False),  # rows not staged
+                                            (17, 4096, 2560, torch.bfloat16, False),  # K slices
+                                            (50, 2560, 9728, torch.float16, False),
+                                            (17, 9216, 960, torch.bfloat16, True)])
+def test_gate_up_silu_entry_past_the_16_row_kernels(M, N, K, act, norm):
+    # where the plain projection runs the tiled kernel (the op then takes the two
+    # launches) the C entry still runs narrow layers, with the projection's sums
+    c = workloads.w8a16_case(M, N, K, seed=M + N, act_dtype=act)
+    g = workloads.device_generator(DEV, 37)
+    x = (torch.randn((M, K), generator=g, device=DEV) * 2).to(act)
+    r = torch.randn((M, K), generator=g, device=DEV).to(act)
+    nw = (1 + 0.1 * torch.randn((K,), generator=g, device=DEV)).to(act)
+    bias = torch.randn((N,), generator=g, device=DEV).to(act)
+    lib = _lib.load()
+    assert lib.sd_w8a16_plan(M, N, K, 0) != 0
+    h, want_res = ops.rmsnorm(x, nw, 1e-6, residual=r) if norm else (x, None)
+    two = ops.silu_mul(ops.w8a16_linear(h, c["w"], c["s"], bias))
+    y = torch.full((M, N // 2), float("nan"), dtype=act, device=DEV)
+    ro = torch.empty_like(x)
+    rc = lib.sd_w8a16_gate_up_silu(x.data_ptr(), K, r.data_ptr() if norm else None, K,
+                                   ro.data_ptr() if norm else None, K,
+                                   nw.data_ptr() if norm else None, 1e-6, c["w"].data_ptr(), K,
+                                   c["s"].data_ptr(), _lib.dtype_code(c["s"].dtype),
+                                   bias.data_ptr(), y.data_ptr(), N // 2, M, N, K,
+                                   _lib.dtype_code(act), _lib.stream_ptr(torch.device(DEV)))
+    _lib.check(rc)
+    assert torch.equal(y, two)
+    assert not norm or torch.equal(ro, want_res)
+    assert torch.equal(ops.w8a16_gate_up_silu(x, c["w"], c["s"], nw if norm else None, 1e-6,
+                                              residual=r if norm else None, bias=bias), two)
+
+
 def test_gate_up_silu_entry_refuses_shapes_off_its_paths():
     # 3 rows (not the row path) of 2064 weight rows (pairs not in whole 16-row tiles)
     c = workloads.w8a16_case(3, 2064, 1024, seed=5)
