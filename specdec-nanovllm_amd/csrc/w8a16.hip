@@ -1228,14 +1228,13 @@ struct RowsPlan {
 
 struct W8Plan {
   int MT, NT, KW, mblocks, groups, grid;
-  int gemm;  // K slices of the many-row kernel (plain calls run it), 0: it stays out
-  int kb;    // 64-column steps per stage: slices start on whole ones
+  sd::W8GemmPlan gemm;  // the many-row kernel (plain calls run it; no slices: it stays out)
   bool narrow;  // too few rows for whole-row waves: gate_up has its SiLU epilogue
 };
 
 W8Plan make_plan(int64_t M, int64_t N, int64_t K, int32_t group) {
   W8Plan pl;
-  pl.gemm = sd::w8a16_gemm_splits(M, N, K, group, &pl.kb);
+  pl.gemm = sd::w8a16_gemm_plan(M, N, K, group);
   // Activation rows in blocks of 16 (MT = 1), 32 (MT = 2) or 64 (MT = 4) along
   // grid.y. Every block streams the whole weight matrix, and a second block
   // only hits L2 while it runs in step with the first: with the weight loads
@@ -1256,7 +1255,7 @@ W8Plan make_plan(int64_t M, int64_t N, int64_t K, int32_t group) {
   // Where plain calls run the many-row kernel, the SiLU and RMSNorm forms keep to its
   // K slices, one wave each (the same sums).
   pl.narrow = nr * pl.mblocks < 8ll * cus && nks >= 4;
-  if (pl.gemm == 1 || (pl.gemm == 0 && !pl.narrow)) {
+  if (pl.gemm.slices == 1 || (pl.gemm.slices == 0 && !pl.narrow)) {
     pl.KW = 1;
     // 16-row groups balance better over the waves (lm_head M = 1: 29.0 vs
     // 30.0 us); from M = 8 up, 32-row groups reuse each activation read twice
@@ -1267,7 +1266,7 @@ W8Plan make_plan(int64_t M, int64_t N, int64_t K, int32_t group) {
     pl.mblocks = static_cast<int>((M + 15) / 16);
     const int64_t tiles = nr * pl.mblocks;
     // (whole 2-step chunks per wave: a partial chunk loads steps nobody uses)
-    pl.KW = pl.gemm > 1 ? pl.gemm
+    pl.KW = pl.gemm.slices > 1 ? pl.gemm.slices
             : tiles * 16 <= 16ll * cus && nks % 32 == 0 ? 16
             : (tiles * 8 <= 16ll * cus && nks % 16 == 0 ? 8 : 4);
   }
@@ -1589,11 +1588,13 @@ bool w8_sizes_ok(int64_t M, int64_t N, int64_t K, int32_t group_size) {
 }  // namespace
 
 extern "C" size_t sd_w8a16_workspace_size(int64_t M, int64_t N, int64_t K, int32_t group_size) {
-  return w8_sizes_ok(M, N, K, group_size) ? sd::w8a16_gemm_workspace(M, N, K, group_size) : 0;
+  if (!w8_sizes_ok(M, N, K, group_size)) return 0;
+  return sd::w8a16_gemm_workspace(sd::w8a16_gemm_plan(M, N, K, group_size), M, N);
 }
 
 extern "C" int64_t sd_w8a16_plan(int64_t M, int64_t N, int64_t K, int32_t group_size) {
-  return w8_sizes_ok(M, N, K, group_size) ? sd::w8a16_gemm_plan_code(M, N, K, group_size) : 0;
+  if (!w8_sizes_ok(M, N, K, group_size)) return 0;
+  return sd::w8a16_gemm_plan_code(sd::w8a16_gemm_plan(M, N, K, group_size));
 }
 
 namespace {
@@ -1699,8 +1700,8 @@ int run_w8a16(const void* x, int64_t x_stride_m, int64_t up, const NormArgs& nor
   p.N = static_cast<int32_t>(N);
   p.K = static_cast<int32_t>(K);
   p.nks = static_cast<int32_t>(K / 64);
-  p.kb = pl.kb;
-  p.nst = p.nks / pl.kb;
+  p.kb = pl.gemm.kb;
+  p.nst = p.nks / pl.gemm.kb;
   p.groups = pl.groups;
   // staged activation rows (wide path): K * 2 bytes + a 16-byte pad per row, so
   // that the 16 rows of a B-operand read start 4 banks apart
@@ -1752,12 +1753,15 @@ int run_w8a16(const void* x, int64_t x_stride_m, int64_t up, const NormArgs& nor
     if (dtype == SD_BF16) return launch_all<__bf16, 0>(p, pp, st);
     return launch_all<_Float16, 0>(p, pp, st);
   }
-  if (pl.gemm > 0 && mode == 0) {
+  if (pl.gemm.slices > 0 && mode == 0) {
     const sd::W8GemmArgs ga{p.x, p.xs, p.w, p.ws, p.scale, p.scale_dtype, p.group, p.bias,
                             p.y, p.ys, p.M, p.N,  p.K,     dtype};
-    int splits = 0;
-    if (sd::w8a16_gemm_fits(ga, workspace, workspace_bytes, &splits))
-      return sd::w8a16_gemm(ga, splits, workspace, st, floor);
+    sd::W8GemmPlan gp = pl.gemm;
+    // without the partial sums' workspace: one slice
+    if (gp.slices > 1 && (!workspace || !sd::aligned16(workspace) ||
+                          workspace_bytes < sd::w8a16_gemm_workspace(gp, M, N)))
+      gp.slices = 1;
+    if (sd::w8a16_gemm_fits(ga, gp)) return sd::w8a16_gemm(ga, gp, workspace, st, floor);
   }
   if (floor) {  // the plain form's plan with the load-only kernels
     if (rows_eligible(p, false)) {

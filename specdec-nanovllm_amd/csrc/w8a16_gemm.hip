@@ -393,24 +393,19 @@ constexpr Cost kCosts[] = {{kT32x64, 0.188, 0.126},  {kT64x64, 0.256, 0.197},  {
                            {kT128x128, 0.63, 0.535}, {kT128x256, 1.0, 1.01},   {kT256x256, 1.43, 1.78}};
 constexpr Cost kCostsGroup[] = {{kT64x128, 0.50, 0.38}, {kT128x128, 1.2, 0.82}};
 
-constexpr int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
-
 // 3, 6 and 12 beside the powers of two: 40 tiles of 2560 rows are 240 workgroups in 6 slices
 // (2560 x 9728, M = 56: 4 slices 18.3 us, 6 slices 15.8; M = 2048 142 -> 114 us with 3).
-struct Plan {
-  Tile tile;
-  int splits;
-};
+constexpr int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
 
 // The tile and the K slices of least estimated time: rounds of workgroups per CU (between
 // the mean and the largest share: workgroups of a CU run together), about three steps to
 // fill and drain a tile, and for several slices the second launch and the partial sums
 // through memory (4.3 TB/s). Checked against the measured best of all tiles and slices at
 // the sizes above: 3% more time in the mean.
-Plan plan_for(int64_t M, int64_t N, int64_t K, int32_t group) {
+sd::W8GemmPlan plan_for(int64_t M, int64_t N, int64_t K, int32_t group) {
   const int64_t nks = K / 64;
   const double cus = sd::device_cus();
-  Plan best{kT64x128, 1};
+  sd::W8GemmPlan best{kT64x128, 1, 1};
   double best_us = 1e30;
   const Cost* costs = group ? kCostsGroup : kCosts;
   const int ncosts = group ? 2 : 9;
@@ -430,7 +425,7 @@ Plan plan_for(int64_t M, int64_t N, int64_t K, int32_t group) {
       if (splits > 1) us += 3.5 + 8.0 * splits * static_cast<double>(M) * static_cast<double>(N) / 4.3e6;
       if (us < best_us) {
         best_us = us;
-        best = Plan{costs[c].tile, splits};
+        best = sd::W8GemmPlan{costs[c].tile, splits, static_cast<int>(kb)};
       }
     }
   return best;
@@ -552,47 +547,32 @@ bool stays_on_16_rows(int64_t M, int64_t N, int64_t K, int32_t group) {
          (M <= 64 && M * K <= 36 * kKi && N >= 96 * kKi && N * K <= 100 * kMi);
 }
 
-int w8a16_gemm_splits(int64_t M, int64_t N, int64_t K, int32_t group, int* kb) {
-  *kb = 1;
-  if (stays_on_16_rows(M, N, K, group)) return 0;
-  const Plan pl = plan_for(M, N, K, group);
-  *kb = kShapes[pl.tile].kb;
-  return pl.splits;
+W8GemmPlan w8a16_gemm_plan(int64_t M, int64_t N, int64_t K, int32_t group) {
+  return stays_on_16_rows(M, N, K, group) ? W8GemmPlan{0, 0, 1} : plan_for(M, N, K, group);
 }
 
-int64_t w8a16_gemm_plan_code(int64_t M, int64_t N, int64_t K, int32_t group) {
-  if (stays_on_16_rows(M, N, K, group)) return 0;
-  const Plan pl = plan_for(M, N, K, group);
-  return pl.splits | static_cast<int64_t>(kShapes[pl.tile].bn) << 8 |
+int64_t w8a16_gemm_plan_code(const W8GemmPlan& pl) {
+  if (pl.slices == 0) return 0;
+  return pl.slices | static_cast<int64_t>(kShapes[pl.tile].bn) << 8 |
          static_cast<int64_t>(kShapes[pl.tile].bm) << 20;
 }
 
-size_t w8a16_gemm_workspace(int64_t M, int64_t N, int64_t K, int32_t group) {
-  int kb;
-  const int splits = w8a16_gemm_splits(M, N, K, group, &kb);
-  if (splits <= 1) return 0;
-  return static_cast<size_t>(splits) * static_cast<size_t>(M) * static_cast<size_t>(pitch_of(N)) * sizeof(float);
+size_t w8a16_gemm_workspace(const W8GemmPlan& pl, int64_t M, int64_t N) {
+  if (pl.slices <= 1) return 0;
+  return static_cast<size_t>(pl.slices) * static_cast<size_t>(M) * static_cast<size_t>(pitch_of(N)) * sizeof(float);
 }
 
-bool w8a16_gemm_fits(const W8GemmArgs& a, const void* workspace, size_t workspace_bytes, int* splits) {
-  int kb;
-  *splits = w8a16_gemm_splits(a.M, a.N, a.K, a.group, &kb);
-  if (*splits == 0) return false;
-  // without the partial sums' workspace: one slice
-  if (*splits > 1 && (!workspace || !aligned16(workspace) ||
-                      workspace_bytes < w8a16_gemm_workspace(a.M, a.N, a.K, a.group)))
-    *splits = 1;
-  // a tile's x rows within 32-bit byte offsets; its LDS; the grid
-  const Tile t = plan_for(a.M, a.N, a.K, a.group).tile;
+bool w8a16_gemm_fits(const W8GemmArgs& a, const W8GemmPlan& pl) {
+  // a tile's x rows within 32-bit byte offsets; the grid; its LDS
+  const Tile t = static_cast<Tile>(pl.tile);
   if (a.xs >= (int64_t{1} << 23)) return false;
-  if (tiles_of(t, a.M, a.N) * *splits > 0x7fffffff) return false;
-  // (one slice instead of the planned ones still has whole stages: nks is a multiple)
-  return !a.group || group_lds(t, a.K, a.group, *splits) <= static_cast<size_t>(device_lds_per_block());
+  if (tiles_of(t, a.M, a.N) * pl.slices > 0x7fffffff) return false;
+  return !a.group || group_lds(t, a.K, a.group, pl.slices) <= static_cast<size_t>(device_lds_per_block());
 }
 
-int w8a16_gemm(const W8GemmArgs& a, int splits, void* workspace, hipStream_t st, bool floor) {
-  const Tile t = plan_for(a.M, a.N, a.K, a.group).tile;
-  const GemmParams p = params(a, splits, workspace);
+int w8a16_gemm(const W8GemmArgs& a, const W8GemmPlan& pl, void* workspace, hipStream_t st, bool floor) {
+  const Tile t = static_cast<Tile>(pl.tile);
+  const GemmParams p = params(a, pl.slices, workspace);
   const int rc = a.dtype == SD_BF16 ? run<__bf16>(t, p, st, floor) : run<_Float16>(t, p, st, floor);
   return rc != SD_OK ? rc : check_launch(floor ? "w8a16 floor" : "w8a16");
 }
