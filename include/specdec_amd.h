@@ -277,8 +277,9 @@ int sd_paged_attention_store(const void* key, int64_t key_stride_tok, int64_t ke
  * Bytes of workspace that sd_w8a16_linear uses for this shape on the current
  * device: the fp32 partial sums of the K slices where more than 16 rows have
  * too few output tiles to fill the device, 0 for every other shape. The scratch
- * must be 16-byte aligned. Without it (NULL or too small) the call still runs,
- * in one slice, and is slower.
+ * must be 16-byte aligned. Without it (NULL or too small) the call still runs
+ * and is slower: on the 16-row kernels with the same sums where output tiles are
+ * few, in one slice (sums in another order) where they are many.
  */
 size_t sd_w8a16_workspace_size(int64_t M, int64_t N, int64_t K, int32_t group_size);
 
@@ -324,7 +325,7 @@ int sd_w8a16_linear(const void* x, int64_t x_stride_m, const int8_t* w, int64_t 
                     void* stream);
 
 /*
- * Measurement twin of sd_w8a16_linear (per-channel scale): the same plan,
+ * Measurement twin of sd_w8a16_linear with its workspace (per-channel scale): the same plan,
  * grid, activation staging, weight loads and prefetch, with every loaded
  * word folded into a register in place of the dequantization, the math and
  * the epilogue. y is not written (a store guarded by a condition on the
@@ -346,7 +347,7 @@ int sd_w8a16_floor(const void* x, int64_t x_stride_m, const int8_t* w, int64_t w
  * models/qwen3.py Qwen3MLP.forward). No counterpart entry in the reference:
  * the fusion saves the SiluAndMul launch and its round trip through memory.
  * The activation equals sd_silu_mul's output bit for bit, so y equals
- * sd_silu_mul followed by sd_w8a16_linear. gate_up: (M, >= 2K) dtype, row
+ * sd_silu_mul followed by sd_w8a16_linear (with its workspace). gate_up: (M, >= 2K) dtype, row
  * stride gate_up_stride_m, sharing no byte with y; the rest as
  * sd_w8a16_linear (no workspace). On the
  * row-streaming path (one or two rows, see sd_w8a16_linear) each wave forms
@@ -368,7 +369,7 @@ int sd_w8a16_silu_linear(const void* gate_up, int64_t gate_up_stride_m, const in
  * gate_up_proj, models/qwen3.py Qwen3DecoderLayer.forward). No counterpart
  * entry in the reference: the fusion saves the RMSNorm launch and its round
  * trip through memory. The normalised row equals sd_rmsnorm's out bit for bit,
- * so y equals sd_rmsnorm followed by sd_w8a16_linear; with a residual,
+ * so y equals sd_rmsnorm followed by sd_w8a16_linear (with its workspace); with a residual,
  * residual_out (may be NULL) receives bf16(x + residual) as sd_rmsnorm's
  * residual_out does, written by one workgroup per row block. residual_out and
  * y may share no byte with x, residual or each other (other workgroups still

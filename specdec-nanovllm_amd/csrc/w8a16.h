@@ -69,6 +69,9 @@ struct W8GemmPlan {
 // 16-row kernels (SiLU, RMSNorm) can add the same slices in the same order. About 0.7 us of
 // host time: a call makes it once.
 W8GemmPlan w8a16_gemm_plan(int64_t M, int64_t N, int64_t K, int32_t group);
+// The same without memory for the partial sums: the 16-row kernels (no slices; they add the
+// shape's slices inside a workgroup, with the same bits) or one slice.
+W8GemmPlan w8a16_gemm_plan_unsliced(int64_t M, int64_t N, int64_t K, int32_t group);
 // The plan as sd_w8a16_plan returns it.
 int64_t w8a16_gemm_plan_code(const W8GemmPlan& pl);
 // Bytes of fp32 partial sums (0 with one slice).

@@ -1757,11 +1757,11 @@ int run_w8a16(const void* x, int64_t x_stride_m, int64_t up, const NormArgs& nor
     const sd::W8GemmArgs ga{p.x, p.xs, p.w, p.ws, p.scale, p.scale_dtype, p.group, p.bias,
                             p.y, p.ys, p.M, p.N,  p.K,     dtype};
     sd::W8GemmPlan gp = pl.gemm;
-    // without the partial sums' workspace: one slice
-    if (gp.slices > 1 && (!workspace || !sd::aligned16(workspace) ||
-                          workspace_bytes < sd::w8a16_gemm_workspace(gp, M, N)))
-      gp.slices = 1;
-    if (sd::w8a16_gemm_fits(ga, gp)) return sd::w8a16_gemm(ga, gp, workspace, st, floor);
+    // (the floor twin writes no partial sums)
+    if (gp.slices > 1 && !floor && (!workspace || !sd::aligned16(workspace) ||
+                                    workspace_bytes < sd::w8a16_gemm_workspace(gp, M, N)))
+      gp = sd::w8a16_gemm_plan_unsliced(M, N, K, group_size);
+    if (gp.slices > 0 && sd::w8a16_gemm_fits(ga, gp)) return sd::w8a16_gemm(ga, gp, workspace, st, floor);
   }
   if (floor) {  // the plain form's plan with the load-only kernels
     if (rows_eligible(p, false)) {

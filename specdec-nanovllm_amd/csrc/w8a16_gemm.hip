@@ -402,7 +402,7 @@ constexpr int kSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
 // fill and drain a tile, and for several slices the second launch and the partial sums
 // through memory (4.3 TB/s). Checked against the measured best of all tiles and slices at
 // the sizes above: 3% more time in the mean.
-sd::W8GemmPlan plan_for(int64_t M, int64_t N, int64_t K, int32_t group) {
+sd::W8GemmPlan plan_for(int64_t M, int64_t N, int64_t K, int32_t group, bool sliced = true) {
   const int64_t nks = K / 64;
   const double cus = sd::device_cus();
   sd::W8GemmPlan best{kT64x128, 1, 1};
@@ -412,7 +412,7 @@ sd::W8GemmPlan plan_for(int64_t M, int64_t N, int64_t K, int32_t group) {
   for (int c = 0; c < ncosts; ++c)
     for (int splits : kSplits) {
       const int64_t kb = kShapes[costs[c].tile].kb;
-      if (splits > 1 && nks < 4 * splits) break;
+      if (splits > 1 && (!sliced || nks < 4 * splits)) break;
       if (nks % kb) break;  // whole stages
       double full = costs[c].full;
       // (a scale table that leaves room for one workgroup per CU)
@@ -549,6 +549,17 @@ bool stays_on_16_rows(int64_t M, int64_t N, int64_t K, int32_t group) {
 
 W8GemmPlan w8a16_gemm_plan(int64_t M, int64_t N, int64_t K, int32_t group) {
   return stays_on_16_rows(M, N, K, group) ? W8GemmPlan{0, 0, 1} : plan_for(M, N, K, group);
+}
+
+// Up to two 16 x 16 output tiles per CU (three per group, where this kernel's step is dearer)
+// the 16-row kernels are faster than one slice here: 2560 x 9728 at M = 48 27.6 us there, 33.5
+// here, at M = 64, 2.5 per CU, 39.8 and 33.8; 4096 x 2560 at M = 32 10.8 and 11.4, 6144 x 2560
+// at M = 17, three per CU, 13.6 and 11.7; in groups of 128 2560 x 4096 at M = 64 31.0 and 41.2,
+// 4096 x 2560 at M = 64, four per CU, 31.6 and 27.1.
+W8GemmPlan w8a16_gemm_plan_unsliced(int64_t M, int64_t N, int64_t K, int32_t group) {
+  const int64_t tiles = (M + 15) / 16 * ((N + 15) / 16);
+  if (stays_on_16_rows(M, N, K, group) || tiles <= (group ? 3 : 2) * device_cus()) return W8GemmPlan{0, 0, 1};
+  return plan_for(M, N, K, group, false);
 }
 
 int64_t w8a16_gemm_plan_code(const W8GemmPlan& pl) {

@@ -423,8 +423,9 @@ def test_gate_up_silu_entry_refuses_shapes_off_its_paths():
 @pytest.mark.parametrize("act", [torch.bfloat16, torch.float16])
 def test_many_rows(M, N, K, gs, act):
     """The tiled kernel at the edges of its tiles, slices and stages, weights over all
-    of int8 (-128 among them), x and y in strided rows, with a bias, against float64
-    and, without the workspace of the K slices, against itself in one slice."""
+    of int8 (-128 among them), x and y in strided rows, with a bias, against float64, and
+    without the workspace of the K slices: on the 16-row kernels with the same sums up to two
+    16 x 16 output tiles per CU (three per group), else in one slice."""
     if gs > K:
         gs = 0
     g = workloads.device_generator(DEV, M + N)
@@ -451,6 +452,9 @@ def test_many_rows(M, N, K, gs, act):
         assert nbytes > 0  # K slices at these sizes
     got = call(torch.empty(nbytes, dtype=torch.uint8, device=DEV) if nbytes else None)
     one = call(None)
+    tiles = -(-M // 16) * -(-N // 16)
+    if not nbytes or tiles <= (3 if gs else 2) * torch.cuda.get_device_properties(0).multi_processor_count:
+        assert torch.equal(got, one)
     assert torch.equal(got, ops.w8a16_linear(x, w, s, bias, group_size=gs))
     assert bool(buf[:, N:].isnan().all())
     rel = 2.0 ** -9 if act == torch.float16 else 2.0 ** -8
@@ -501,7 +505,8 @@ def test_two_rows_on_wide_matrices_stay_on_the_tiled_kernel():
 
 # ----------------------------------------------------- measurement twins
 @pytest.mark.parametrize("M,N,K", [(1, 151936, 1024), (7, 151936, 1024), (56, 151936, 1024),
-                                   (1, 4096, 1024), (16, 1024, 3072), (56, 6144, 1024)])
+                                   (1, 4096, 1024), (16, 1024, 3072), (56, 6144, 1024),
+                                   (17, 2560, 9728), (56, 2560, 9728), (56, 19456, 2560)])
 @pytest.mark.parametrize("act", [torch.float16, torch.bfloat16])
 def test_floor_twin_runs_the_plan_and_writes_nothing(M, N, K, act):
     # sd_w8a16_floor: the same plan with no math leaves the output untouched
