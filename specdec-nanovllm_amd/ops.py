@@ -319,9 +319,10 @@ def w8a16_linear(x: torch.Tensor, qweight: torch.Tensor, scale: torch.Tensor,
                 _lib.stream_ptr(dev))
         _lib.check(rc)
         return y.view(*x.shape[:-1], N)
-    ws_bytes = lib.sd_w8a16_workspace_size(M, N, K, int(group_size))
-    ws = _workspace(ws_bytes, dev)
     with _lib.on_device(dev):
+        # the plan (and so the workspace) depends on the device's compute units
+        ws_bytes = lib.sd_w8a16_workspace_size(M, N, K, int(group_size))
+        ws = _workspace(ws_bytes, dev)
         rc = lib.sd_w8a16_linear(
             x2.data_ptr(), x2.stride(0), qw.data_ptr(), qw.stride(0),
             sc.data_ptr(), _lib.dtype_code(sc.dtype), int(group_size), _ptr(b),

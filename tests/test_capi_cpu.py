@@ -2,6 +2,7 @@
 include/specdec_amd.h declares, the ctypes table matches the header's
 parameter counts, and argument validation (which returns before any HIP call)
 reports the reference's error kinds. No kernel is launched here."""
+import contextlib
 import ctypes
 import os
 import re
@@ -146,6 +147,35 @@ def test_ops_refuse_cpu_tensors():
     with pytest.raises(RuntimeError, match="ROCm GPU"):
         ops.w8a16_linear(torch.zeros((1, 64), dtype=torch.float16),
                          torch.zeros((8, 64), dtype=torch.int8), torch.ones(8))
+
+
+def test_w8a16_linear_asks_for_its_workspace_on_the_tensors_device(monkeypatch):
+    # the plan, and so the size, follows the current device's compute units
+    current, seen = [0], {}
+
+    @contextlib.contextmanager
+    def on_device(dev):
+        current.append(dev.index)
+        yield
+        current.pop()
+
+    class Lib:
+        def sd_w8a16_workspace_size(self, *sizes):
+            seen["size"] = current[-1]
+            return 64
+
+        def sd_w8a16_linear(self, *args):
+            seen["linear"] = current[-1]
+            return 0
+
+    monkeypatch.setattr(_lib, "require_device", lambda *t: torch.device("cuda", 1))
+    monkeypatch.setattr(_lib, "load", Lib)
+    monkeypatch.setattr(_lib, "on_device", on_device)
+    monkeypatch.setattr(_lib, "stream_ptr", lambda dev: None)
+    monkeypatch.setattr(ops, "_workspace", lambda n, dev: torch.empty(n, dtype=torch.uint8))
+    ops.w8a16_linear(torch.zeros((32, 64), dtype=torch.bfloat16), torch.zeros((8, 64), dtype=torch.int8),
+                     torch.ones(8), out=torch.empty((32, 8), dtype=torch.bfloat16))
+    assert seen == {"size": 1, "linear": 1}
 
 
 @pytest.mark.skipif(torch.cuda.device_count() > 0,
