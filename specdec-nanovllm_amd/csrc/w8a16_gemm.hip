@@ -367,11 +367,12 @@ size_t table_bytes(Tile t, int64_t K, int32_t group, int splits) {
   return static_cast<size_t>(kShapes[t].bn) * static_cast<size_t>((per + spg - 2) / spg + 1) * sizeof(float);
 }
 
-// Per-group tiles: stages, their bytes with the table.
-constexpr int kGroupStages64 = 3, kGroupStages128 = 2;
-size_t group_lds(Tile t, int64_t K, int32_t group, int splits) {
-  const size_t stages = t == kT64x128 ? kGroupStages64 : kGroupStages128;
-  return stages * (kShapes[t].bm * 128 + kShapes[t].bn * 64) + table_bytes(t, K, group, splits);
+// The per-group tile: its stages, their bytes with the table.
+constexpr Tile kGroupTile = kT64x128;
+constexpr int kGroupStages = 3;
+size_t group_lds(int64_t K, int32_t group, int splits) {
+  return static_cast<size_t>(kGroupStages) * (kShapes[kGroupTile].bm * 128 + kShapes[kGroupTile].bn * 64) +
+         table_bytes(kGroupTile, K, group, splits);
 }
 
 // What a tile costs, in microseconds per 64-column step, measured at 256 CUs (M 17 - 6896;
@@ -383,7 +384,7 @@ size_t group_lds(Tile t, int64_t K, int32_t group, int splits) {
 // are for widths whose 64-row tiles just miss a whole number of workgroups per CU: 19456 x 2560
 // is 304 tiles of 64 rows, 203 of 96 (weights from HBM: M = 56 21.7 -> 18.6 us, M = 100 64 x 256
 // 29.9, 64 x 80 25.0); five stages instead of three measured 2 - 5% slower there. Per group the step sums
-// and scales come on top, and the tiles stop at 64 x 64 outputs per wave.
+// and scales come on top (a 128 x 128 tile took 0.82 us, more than two of 64 x 128).
 struct Cost {
   Tile tile;
   double alone, full;
@@ -391,7 +392,7 @@ struct Cost {
 constexpr Cost kCosts[] = {{kT32x64, 0.188, 0.126},  {kT64x64, 0.256, 0.197},  {kT64x80, 0.307, 0.23},
                            {kT64x96, 0.303, 0.30},  {kT64x128, 0.44, 0.36},   {kT64x256, 0.50, 0.68},
                            {kT128x128, 0.63, 0.535}, {kT128x256, 1.0, 1.01},   {kT256x256, 1.43, 1.78}};
-constexpr Cost kCostsGroup[] = {{kT64x128, 0.50, 0.38}, {kT128x128, 1.2, 0.82}};
+constexpr Cost kCostsGroup[] = {{kGroupTile, 0.50, 0.38}};
 
 // 3, 6 and 12 beside the powers of two: 40 tiles of 2560 rows are 240 workgroups in 6 slices
 // (2560 x 9728, M = 56: 4 slices 18.3 us, 6 slices 15.8; M = 2048 142 -> 114 us with 3).
@@ -408,7 +409,7 @@ sd::W8GemmPlan plan_for(int64_t M, int64_t N, int64_t K, int32_t group, bool sli
   sd::W8GemmPlan best{kT64x128, 1, 1};
   double best_us = 1e30;
   const Cost* costs = group ? kCostsGroup : kCosts;
-  const int ncosts = group ? 2 : 9;
+  const int ncosts = group ? 1 : 9;
   for (int c = 0; c < ncosts; ++c)
     for (int splits : kSplits) {
       const int64_t kb = kShapes[costs[c].tile].kb;
@@ -416,7 +417,7 @@ sd::W8GemmPlan plan_for(int64_t M, int64_t N, int64_t K, int32_t group, bool sli
       if (nks % kb) break;  // whole stages
       double full = costs[c].full;
       // (a scale table that leaves room for one workgroup per CU)
-      if (group && group_lds(costs[c].tile, K, group, splits) > 80 * 1024) full = costs[c].alone;
+      if (group && group_lds(K, group, splits) > 80 * 1024) full = costs[c].alone;
       const double n = static_cast<double>(tiles_of(costs[c].tile, M, N)) * splits / cus;
       const double whole = static_cast<double>(static_cast<int64_t>(n)) + (n > static_cast<int64_t>(n) ? 1 : 0);
       const double shared = n > 1 ? 0.5 * (n + whole) * full : n * full;
@@ -453,8 +454,7 @@ int launch(GemmParams p, Tile t, hipStream_t st) {
 template <typename T, bool PG, bool FLOOR>
 int launch_tile(Tile t, const GemmParams& p, hipStream_t st) {
   if constexpr (PG) {
-    if (t == kT64x128) return launch<T, 1, 4, 4, 2, kGroupStages64, 1, 2, true, FLOOR>(p, t, st);
-    return launch<T, 2, 2, 4, 4, kGroupStages128, 1, 2, true, FLOOR>(p, t, st);
+    return launch<T, 1, 4, 4, 2, kGroupStages, 1, 2, true, FLOOR>(p, t, st);
   } else {
     switch (t) {
       case kT32x64: return launch<T, 1, 4, 2, 1, 3, 2, 4, false, FLOOR>(p, t, st);
@@ -578,7 +578,7 @@ bool w8a16_gemm_fits(const W8GemmArgs& a, const W8GemmPlan& pl) {
   const Tile t = static_cast<Tile>(pl.tile);
   if (a.xs >= (int64_t{1} << 23)) return false;
   if (tiles_of(t, a.M, a.N) * pl.slices > 0x7fffffff) return false;
-  return !a.group || group_lds(t, a.K, a.group, pl.slices) <= static_cast<size_t>(device_lds_per_block());
+  return !a.group || group_lds(a.K, a.group, pl.slices) <= static_cast<size_t>(device_lds_per_block());
 }
 
 int w8a16_gemm(const W8GemmArgs& a, const W8GemmPlan& pl, void* workspace, hipStream_t st, bool floor) {

@@ -131,6 +131,7 @@ def test_w8a16_routes_to_tiles(M, N, K, group):
     plan = _lib.load().sd_w8a16_plan(M, N, K, group)
     assert plan & 0xff in (1, 2, 3, 4, 6, 8, 12, 16)  # K slices
     assert (plan >> 8) & 0xfff in (64, 80, 96, 128, 256) and plan >> 20 in (32, 64, 128, 256)
+    assert group == 0 or (plan >> 20, plan >> 8 & 0xfff) == (64, 128)  # the per-group tile
 
 
 def test_ops_refuse_cpu_tensors():
