@@ -405,29 +405,38 @@ def test_gate_up_silu_entry_refuses_shapes_off_its_paths():
 
 
 # ------------------------------------------------------------- many rows
-@pytest.mark.parametrize("M,N,K,gs", [(17, 9001, 1024, 0),      # two-step stages, a ragged last tile
-                                      (33, 20010, 640, 0),      # one row into a second 32-row tile
-                                      (40, 9000, 1088, 0),      # an odd number of steps
-                                      (65, 16400, 640, 0),      # one row into a second 64-row tile
-                                      (63, 19427, 640, 0),      # 64 x 96 tiles: waves that load the last KB twice
-                                      (100, 19456, 192, 0),     # 64 x 80 tiles
-                                      (125, 19421, 640, 0),     # the same, ragged
-                                      (18, 2570, 9728, 0),      # 12 K slices, a remainder in each
-                                      (129, 1030, 9728, 0),     # K slices, added by the second launch
-                                      (200, 1030, 2048, 128),   # the same per group, N % 4 != 0
-                                      (300, 6144, 1024, 64),    # one scale per step
-                                      (257, 24200, 192, 0),     # three steps
-                                      (1025, 12290, 64, 0),     # a single step, odd outputs
-                                      (2049, 8200, 256, 0),     # 128 x 256 and 256 x 256 tiles
-                                      (4097, 9728, 128, 256)])
+# tile: (activation rows, weight rows, K slices) of the plan at 256 compute units, None: the
+# 16-row kernels
+@pytest.mark.parametrize("M,N,K,gs,tile", [
+    (17, 9001, 1024, 0, (32, 64, 1)),      # two-step stages, a ragged last tile
+    (33, 20010, 640, 0, (64, 96, 1)),      # one M tile: waves that load the last KB twice
+    (65, 9010, 1024, 0, (32, 64, 1)),      # one row into a third 32-row tile
+    (40, 9000, 1088, 0, (64, 128, 1)),     # an odd number of steps
+    (65, 16400, 640, 0, (64, 80, 1)),      # one row into a second 64-row tile
+    (63, 19427, 640, 0, (64, 96, 1)),
+    (100, 19456, 192, 0, None),
+    (100, 19456, 640, 0, (64, 80, 1)),
+    (125, 19421, 640, 0, (64, 80, 1)),     # the same, ragged
+    (100, 2570, 9728, 0, (64, 64, 6)),
+    (18, 2570, 9728, 0, (32, 64, 12)),     # a remainder in each slice
+    (129, 1030, 9728, 0, (32, 64, 6)),     # K slices, added by the second launch
+    (200, 1030, 2048, 128, (64, 128, 6)),  # the same per group, N % 4 != 0
+    (300, 6144, 1024, 64, (64, 128, 1)),   # one scale per step
+    (4097, 1030, 256, 128, (64, 128, 1)),  # 65 M tiles, two groups
+    (257, 24200, 192, 0, (64, 256, 1)),    # three steps
+    (1025, 12290, 64, 0, (256, 256, 1)),   # a single step, odd outputs
+    (2049, 8200, 256, 0, (128, 128, 1)),
+    (2049, 9728, 128, 0, (128, 256, 1)),
+    (4097, 9728, 128, 0, (256, 256, 1))])
 @pytest.mark.parametrize("act", [torch.bfloat16, torch.float16])
-def test_many_rows(M, N, K, gs, act):
+def test_many_rows(M, N, K, gs, tile, act):
     """The tiled kernel at the edges of its tiles, slices and stages, weights over all
     of int8 (-128 among them), x and y in strided rows, with a bias, against float64, and
     without the workspace of the K slices: on the 16-row kernels with the same sums up to two
     16 x 16 output tiles per CU (three per group), else in one slice."""
-    if gs > K:
-        gs = 0
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        plan = _lib.load().sd_w8a16_plan(M, N, K, gs)
+        assert (plan and (plan >> 20, plan >> 8 & 0xfff, plan & 0xff)) == (tile or 0)
     g = workloads.device_generator(DEV, M + N)
     w = torch.randint(-128, 128, (N, K), generator=g, device=DEV, dtype=torch.int32).to(torch.int8)
     shape = (N, K // gs) if gs else (N,)
