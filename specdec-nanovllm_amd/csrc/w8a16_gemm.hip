@@ -5,8 +5,11 @@
 //   y[m, n] = scale[n] * sum_k x[m, k] * w[n, k] (+ bias[n])           per channel
 //   y[m, n] = sum_g scale[n, g] * sum_{k in g} x[m, k] * w[n, k] (+ bias)  per group
 //
-// Bound: the matrix cores (2 M N K operations against N K + 2 M (N + K) bytes) from
-// about 200 rows up, HBM below. Layout of one step (64 columns of K):
+// Bound by operations (2 M N K against N K + 2 M (N + K) bytes) from about 200 rows up, by
+// bytes below. Counters (bf16): 4096 x 19456 x 2560, 256 x 256 tiles, 370 us: MFMA busy 52% of
+// the SIMD cycles, vector issue 37%; 56 x 19456 x 2560, 64 x 96 tiles, 22 us: MFMA 10%, vector
+// 12%, 52% of the wave cycles waiting at under one wave per SIMD; 56 x 151936 x 1024, 64 x 128
+// tiles, 50 us: 15%, 21%, 42%. Layout of one step (64 columns of K):
 //  * x rows (128 B) and weight rows (64 B) go from HBM / L2 straight into LDS
 //    (global_load_lds, 16 B per lane, no registers); the 16-byte units of a row are
 //    permuted by the global address of each lane, so that the 16 lanes of an operand read
@@ -59,6 +62,7 @@ template <int N> __device__ __forceinline__ void wait_barrier() {
 // unit of 16 x rows, or of the weight rows 4 NT j + i (i, j < 4): with two 128-byte x rows
 // (four 64-byte weight rows) to a 256-byte bank row when KB is 1, whole bank rows (two
 // 128-byte ones) when it is 2, the 16 lanes then cover 16 different 16-byte slots.
+// (SQ_LDS_BANK_CONFLICT counts none with KB = 2, but 4 cycles per read with KB = 1.)
 template <int KB> __device__ __forceinline__ int x_swizzle(int r) { return KB == 1 ? (r >> 1) & 7 : r & 15; }
 template <int KB, int NT> __device__ __forceinline__ int w_swizzle(int r) {
   const int j = (r / (4 * NT)) & 3;
@@ -149,8 +153,9 @@ void w8a16_gemm_kernel(GemmParams p) {
 
   const int nb = n0 + wn * NT * 16 + lg * 4 * NT;  // first of this lane's 4 NT outputs per row
 
-  // ---- per-channel scales (and bias) of this lane's outputs, ahead of the loop; per
-  //      group: the slice's table in LDS after the stages, [group][BN] in fp32
+  // ---- per-channel scales of this lane's outputs, ahead of the loop (one after another:
+  //      load_scale branches on their type; the bias follows the loop); per group: the
+  //      slice's table in LDS after the stages, [group][BN] in fp32
   float sc[PG ? 1 : NT][4];
   float* tab = reinterpret_cast<float*>(sm + S * SB);
   const int spg = PG ? a.group / 64 : 1;           // steps per group
@@ -445,9 +450,9 @@ int launch(GemmParams p, Tile t, hipStream_t st) {
   return SD_OK;
 }
 
-// Waves per tile: the small tiles are bound by instruction issue (one wave issues a vector
-// instruction every 8 cycles or so), so they take 16 weight rows per wave and several
-// workgroups per CU, and read 128-byte pieces of a row. Two stages where the tiles are many:
+// Waves per tile: the waves of the small tiles wait about half of their cycles, so these take
+// 16 weight rows per wave and several workgroups per CU, and read 128-byte pieces of a row.
+// (The fp16 128 x 256 instance spills two registers under its four waves per SIMD.) Two stages where the tiles are many:
 // more workgroups per CU measured better than more stages (128 x 128 at 4096 x 19456 x 2560
 // 398 against 424 us), three or four where loads wait for HBM (64 x 128 at M = 56 of
 // 19456 x 2560 23 us with two, 20 with four, 24 with eight and one workgroup per CU).
