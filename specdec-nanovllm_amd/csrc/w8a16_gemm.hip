@@ -553,7 +553,11 @@ bool stays_on_16_rows(int64_t M, int64_t N, int64_t K, int32_t group) {
 }
 
 W8GemmPlan w8a16_gemm_plan(int64_t M, int64_t N, int64_t K, int32_t group) {
-  return stays_on_16_rows(M, N, K, group) ? W8GemmPlan{0, 0, 1} : plan_for(M, N, K, group);
+  constexpr W8GemmPlan kNone{0, 0, 1};
+  if (stays_on_16_rows(M, N, K, group)) return kNone;
+  const W8GemmPlan pl = plan_for(M, N, K, group);
+  // a launch takes fewer than 2^32 work-items; a workgroup has up to 512
+  return tiles_of(static_cast<Tile>(pl.tile), M, N) * pl.slices < (int64_t{1} << 23) ? pl : kNone;
 }
 
 // Up to two 16 x 16 output tiles per CU (three per group, where this kernel's step is dearer)
@@ -579,10 +583,8 @@ size_t w8a16_gemm_workspace(const W8GemmPlan& pl, int64_t M, int64_t N) {
 }
 
 bool w8a16_gemm_fits(const W8GemmArgs& a, const W8GemmPlan& pl) {
-  // a tile's x rows within 32-bit byte offsets; the grid; its LDS
-  const Tile t = static_cast<Tile>(pl.tile);
+  // a tile's x rows within 32-bit byte offsets; its LDS
   if (a.xs >= (int64_t{1} << 23)) return false;
-  if (tiles_of(t, a.M, a.N) * pl.slices > 0x7fffffff) return false;
   return !a.group || group_lds(a.K, a.group, pl.slices) <= static_cast<size_t>(device_lds_per_block());
 }
 

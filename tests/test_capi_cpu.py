@@ -116,7 +116,8 @@ def test_workspace_queries():
     (192, 1024, 1024, 0), (512, 256, 1024, 0), (256, 256, 2048, 0), (256, 256, 3072, 0),
     (256, 1024, 1024, 128), (64, 6144, 1024, 128), (32, 12288, 1024, 128), (512, 64, 2048, 128),
     (17, 151936, 64, 0), (32, 65536, 512, 0), (32, 151936, 1024, 0), (64, 100000, 512, 0),
-    (48, 100000, 768, 0), (24, 65536, 512, 128), (32, 262144, 128, 128)])
+    (48, 100000, 768, 0), (24, 65536, 512, 128), (32, 262144, 128, 128),
+    (1 << 30, 64, 128, 0)])  # more work-items than a launch takes
 def test_w8a16_routes_to_the_16_row_kernels(M, N, K, group):
     # sizes that measured faster on them than in tiles
     assert _lib.load().sd_w8a16_plan(M, N, K, group) == 0
