@@ -172,6 +172,9 @@ def test_errors():
                                           (33, 2560, 4096, 0, torch.float16),
                                           (200, 1030, 2048, 128, torch.bfloat16),
                                           (640, 4096, 576, 0, torch.bfloat16),
+                                          (512, 2560, 9728, 0, torch.bfloat16),  # 2
+                                          (17, 2560, 4096, 0, torch.float16),    # 8
+                                          (153, 81, 11392, 0, torch.bfloat16),   # 16
                                           (3, 33000, 1024, 0, torch.bfloat16),
                                           (20, 33000, 1024, 128, torch.float16),
                                           (40, 33000, 1024, 0, torch.bfloat16),
@@ -423,6 +426,8 @@ def test_gate_up_silu_entry_refuses_shapes_off_its_paths():
     (200, 1030, 2048, 128, (64, 128, 6)),  # the same per group, N % 4 != 0
     (300, 6144, 1024, 64, (64, 128, 1)),   # one scale per step
     (4097, 1030, 256, 128, (64, 128, 1)),  # 65 M tiles, two groups
+    # in one slice (no workspace) the scale table is too large: the 16-row kernels
+    (200, 2056, 16384, 64, (64, 128, 6)),
     (257, 24200, 192, 0, (64, 256, 1)),    # three steps
     (1025, 12290, 64, 0, (256, 256, 1)),   # a single step, odd outputs
     (2049, 8200, 256, 0, (128, 128, 1)),
