@@ -1339,6 +1339,12 @@ constexpr size_t w8_static_lds() {
          static_cast<size_t>(KW > 1 ? KW - 1 : 1) * (NT * MT * 4) * 64 * 4;
 }
 
+int norm_does_not_fit(int rows, int K) {
+  sd::set_error("w8a16_rmsnorm: the activation block (%d rows of K = %d) does not fit the "
+                "staging LDS", rows, K);
+  return SD_ERR_UNSUPPORTED;
+}
+
 template <typename T, int MT, int NT, int KW, bool PG, int MODE, bool FLOOR = false,
           bool PAIRED = false>
 int launch_k(const W8Params& p, dim3 grid, hipStream_t st) {
@@ -1385,9 +1391,7 @@ int launch_k(const W8Params& p, dim3 grid, hipStream_t st) {
   }
   if constexpr (MODE == 2) {
     // the norm needs the rows staged: no register form
-    sd::set_error("w8a16_rmsnorm: the activation block (%d rows of K = %d) does not fit the "
-                  "staging LDS", static_cast<int>(p.M < MT * 16 ? p.M : MT * 16), p.K);
-    return SD_ERR_UNSUPPORTED;
+    return norm_does_not_fit(static_cast<int>(p.M < MT * 16 ? p.M : MT * 16), p.K);
   } else {
     auto kern = w8a16_kernel<T, MT, NT, KW, U, PG, false, 2, false, MODE, NWV, FLOOR, PAIRED>;
     // exactly one resident set of workgroups over all activation blocks (a
@@ -1415,6 +1419,9 @@ int launch_kw(const W8Params& p, const W8Plan& pl, dim3 grid, hipStream_t st) {
       case 4 * 8 + 2: return launch_k<T, 4, 2, 1, PG, MODE, FLOOR>(p, grid, st);
       default: return launch_k<T, 2, 2, 1, PG, MODE, FLOOR>(p, grid, st);
     }
+  } else if constexpr (MODE == 2 && (KW == 6 || KW == 12)) {
+    // (more than 16 rows of K >= 1536: a slice is at least four steps)
+    return norm_does_not_fit(16, p.K);
   } else {
     if (p.pair > 0) {  // gate_up with the SiLU epilogue: gate and up tile per group
       if constexpr (!PG && MODE != 1 && !FLOOR) return launch_k<T, 1, 2, KW, PG, MODE>(p, grid, st);
